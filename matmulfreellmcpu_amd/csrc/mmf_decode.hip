@@ -116,17 +116,17 @@ void k_decode(DecArgs a) {
   const float* const nw0 = a.p[0].normwT;
   const float* const nw1 = a.p[1].normwT;
   const float* const nw2 = a.p[2].normwT;
-  const float* const ax = a.x;
+  const float* ax = a.x;
   const float* const aembT = a.embT;
-  const float* const ax2 = a.x2;
+  const float* ax2 = a.x2;
   const float* const apre = a.pre_w;
   const float* const alb = a.lb;
-  const float* const ahin = a.hin;
-  float* const astate = a.state;
-  float* const arecur = a.recur;
-  float* const agout = a.gout;
-  float* const aout = a.out;
-  unsigned long long* const akeys = a.keys;
+  const float* ahin = a.hin;
+  float* astate = a.state;
+  float* arecur = a.recur;
+  float* agout = a.gout;
+  float* aout = a.out;
+  unsigned long long* akeys = a.keys;
   int64_t* const ahist = a.hist;
   int32_t* const ahist_pos = a.hist_pos;
   const int awg = a.wgroups, aoLc = a.oLc, aoK8 = a.oK8, aH = a.H, avocab = a.vocab, ankeys = a.nkeys,
@@ -151,6 +151,21 @@ void k_decode(DecArgs a) {
 #undef MMF_PIN_BASE
   const int Ww = W4 ? 2 * Wc : Wc;  // slab words per chain
   const int W = 8 * Lc + 8;  // floats of a chain-transposed vector in global memory
+  const int sb = blockIdx.y;  // the stream: its vectors follow the first stream's
+  if (sb > 0) {
+    const size_t oi = static_cast<size_t>(sb) * W, oo = static_cast<size_t>(sb) * (8 * aoLc + 8);
+    if (ax) ax += oi;
+    if (KIND == kO) ax2 += oi;
+    if (KIND == kO || KIND == kDown) ahin += oo;
+    if (KIND == kIFG) {
+      astate += static_cast<size_t>(sb) * aH;
+      arecur += oo;
+      agout += oo;
+    }
+    if (aout) aout += (KIND == kLM) ? static_cast<size_t>(sb) * avocab
+                      : (KIND == kDown && a.out_nat) ? static_cast<size_t>(sb) * gN : oo;
+    if (KIND == kLM && akeys) akeys += static_cast<size_t>(sb) * kLMBlocks;
+  }
   const int F4 = W / 4;  // float4s of a chain-transposed vector
   // LDS copies pad each chain row by 16 bytes so that the 8 chain lanes of a wave read
   // different banks: float rows LS floats apart, int8 plane rows LQ bytes apart.
@@ -195,7 +210,9 @@ void k_decode(DecArgs a) {
 
   // layer 0: the token is the argmax over the previous lm_head's per-block keys
   int64_t tok = 0;
-  if (KIND == kIFG && ax == nullptr) {
+  if (KIND == kIFG && ax == nullptr && a.tokens) {
+    tok = a.tokens[sb];
+  } else if (KIND == kIFG && ax == nullptr) {
     unsigned long long best = 0ull;
     for (int e0 = tid; e0 < ankeys; e0 += 8 * BS) {  // 8 keys per thread in flight at once
       unsigned long long k[8];
@@ -656,7 +673,7 @@ void k_decode(DecArgs a) {
       agout[p] = v2;
       if (aout) aout[p] = src[0][p];  // layer 0: the embedding row becomes h
     } else if (KIND == kO || KIND == kDown) {
-      aout[p] = e_hin + val;
+      aout[(KIND == kDown && a.out_nat) ? o : p] = e_hin + val;
     } else {  // kGate
       aout[p] = swiglu_of(val, v1, o >= (nout & ~7));
     }
@@ -723,12 +740,15 @@ __global__ __launch_bounds__(64 * KindTraits<KIND>::NM) void k_decf(const float*
   const float pinv = Pa.inv_scale_w;
   const float aeps = a.eps;
   const int nout = gN;
-  const int W = 8 * S::Lc + 8;
+  constexpr int W = 8 * S::Lc + 8;
+  const int sb = blockIdx.y;  // the stream: its input vectors follow the first stream's
 
   // layer 0: the token is the argmax over the previous lm_head's per-block keys (every wave
-  // reduces all keys itself)
-  const float* src0 = xin;
-  if (KIND == kIFG && xin == nullptr) {
+  // reduces all keys itself), or the caller's
+  const float* src0 = xin + static_cast<size_t>(sb) * W;
+  if (KIND == kIFG && xin == nullptr && a.tokens) {
+    src0 = a.embT + static_cast<size_t>(a.tokens[sb]) * W;
+  } else if (KIND == kIFG && xin == nullptr) {
     const unsigned long long* keys = a.keys;
     const int nkeys = a.nkeys;
     unsigned long long best = 0ull;
@@ -779,7 +799,7 @@ __global__ __launch_bounds__(64 * KindTraits<KIND>::NM) void k_decf(const float*
     load_seg<RC>(src0, lane, xs, xt);
   }
   if constexpr (ST1) load_seg<RC>(prew, lane, ws, wt);
-  if constexpr (KIND == kO) load_seg<RC>(xg, lane, gs, gt);
+  if constexpr (KIND == kO) load_seg<RC>(xg + static_cast<size_t>(sb) * W, lane, gs, gt);
   // kDown at RC >= 22: row, norm weight and slab words would be 3 RC > 63 loads in flight,
   // and the wave would stall issuing them until the first ones return; the norm weight's
   // loads are issued in the middle of the norm chain instead (they are needed after it)
@@ -808,13 +828,18 @@ __global__ __launch_bounds__(64 * KindTraits<KIND>::NM) void k_decf(const float*
   const int o = 8 * static_cast<int>(blockIdx.x) + ol;
   const bool epi = mi == 0 && j == 0 && o < nout;
   const int po = epi ? (KIND == kOp ? o : ((o < a.oK8) ? (o & 7) * a.oLc + (o >> 3) : 8 * a.oLc + (o - a.oK8))) : 0;
+  // this stream's outputs (kIFG: state and the H-long vectors; kO, kDown: one vector)
+  const size_t so = static_cast<size_t>(sb) * (8 * a.oLc + 8);
+  const bool nat = KIND == kDown && a.out_nat;
+  float* const state_b = (KIND == kIFG) ? a.state + static_cast<size_t>(sb) * a.H : nullptr;
+  float* const out_b = (KIND == kOp || (KIND == kIFG && !a.out)) ? a.out : a.out + (nat ? static_cast<size_t>(sb) * gN : so);
   float e_lb = 0.0f, e_st = 0.0f, e_hin = 0.0f;
   if (epi) {
     if (KIND == kIFG) {
       if (a.lb) e_lb = a.lb[o];
-      e_st = a.state[o];
+      e_st = state_b[o];
     }
-    if (KIND == kO || KIND == kDown) e_hin = a.hin[po];
+    if (KIND == kO || KIND == kDown) e_hin = a.hin[so + po];
   }
   // FixedQ510: the output's 128 * rowsum term (lane j == 0 of every matrix), fetched now
   const int32_t e_rs = (MODE == kFixed && j == 0 && o < nout) ? 128 * Pa.rowsum[o] : 0;
@@ -1026,15 +1051,15 @@ __global__ __launch_bounds__(64 * KindTraits<KIND>::NM) void k_decf(const float*
     if (a.lb) f = __builtin_fmaf(1.0f - e_lb, f, e_lb);
     const float in = swiglu_of(val, 1.0f - f, tl);
     const float s = __builtin_fmaf(f, e_st, in);
-    a.state[o] = s;
-    a.recur[p] = silu_of(s, tl);
-    a.gout[p] = v2;
-    if (a.out) a.out[p] = src0[p];  // layer 0: the embedding row becomes h
+    state_b[o] = s;
+    a.recur[so + p] = silu_of(s, tl);
+    a.gout[so + p] = v2;
+    if (out_b) out_b[p] = src0[p];  // layer 0: the embedding row becomes h
   } else if (KIND == kOp) {
-    a.out[p] = val;
+    out_b[p] = val;
     if (MODE != kFloat && a.acc) a.acc[p] = stot;
   } else {  // kO, kDown
-    a.out[p] = e_hin + val;
+    out_b[nat ? o : p] = e_hin + val;
   }
 }
 
@@ -1042,7 +1067,7 @@ template <int MODE, int KIND, int RC>
 hipError_t decf_rc(const DecArgs& a, hipStream_t s) {
   using S = DecfShape<MODE, KIND, RC>;
   const size_t lds = (static_cast<size_t>(S::NM) * S::SLICE + S::NM * 8) * sizeof(float);
-  const int grid = (a.p[0].g.N + 7) / 8;
+  const dim3 grid((a.p[0].g.N + 7) / 8, a.streams > 1 ? a.streams : 1);
   const float* prew = (KIND == kDown || KIND == kOp) ? nullptr : a.pre_w;
   const float* xg = (KIND == kO) ? a.x2 : nullptr;
   return launch_k(k_decf<MODE, KIND, RC>, grid, 64 * S::NM, lds, s, a.x, prew, xg, a.p[0].normwT, a.p[1].normwT,
@@ -1115,7 +1140,7 @@ constexpr int kParts = (MODE == kFloat) ? 1 : ((KIND == kO || KIND == kDown) ? 4
 constexpr int nv_for(int F4, int BS) { return F4 <= 2 * BS ? 2 : (F4 <= 4 * BS ? 4 : (F4 <= 8 * BS ? 8 : 16)); }
 
 template <int MODE, int KIND, int KS, int RC, bool W4>
-hipError_t dec_rc(const DecArgs& a, size_t lds, int grid, hipStream_t s) {
+hipError_t dec_rc(const DecArgs& a, size_t lds, dim3 grid, hipStream_t s) {
   constexpr int BS = kBlock * KindTraits<KIND>::NM * KS;
   constexpr int F4 = (8 * 32 * RC + 8) / 4;  // float4s of a chain-transposed vector
   static_assert(F4 <= 16 * BS, "row too long for the block layout");
@@ -1123,7 +1148,7 @@ hipError_t dec_rc(const DecArgs& a, size_t lds, int grid, hipStream_t s) {
 }
 
 template <int MODE, int KIND, int KS, bool W4>
-hipError_t dec_ks(const DecArgs& a, size_t lds, int grid, hipStream_t s) {
+hipError_t dec_ks(const DecArgs& a, size_t lds, dim3 grid, hipStream_t s) {
   constexpr int BS = kBlock * KindTraits<KIND>::NM * KS;
   const int Lc = a.p[0].g.Lc;
   if (Lc % 32 == 0) {  // register chains at the model widths: H 1024/2048/2560, I 2816/5632/6912
@@ -1152,7 +1177,7 @@ hipError_t dec_ks(const DecArgs& a, size_t lds, int grid, hipStream_t s) {
 }
 
 template <int MODE, int KIND>
-hipError_t dec_kind(const DecArgs& a, size_t lds, int grid, bool w4, hipStream_t s) {
+hipError_t dec_kind(const DecArgs& a, size_t lds, dim3 grid, bool w4, hipStream_t s) {
   if constexpr (KIND == kLM) {
     switch (a.wgroups) {  // one part per group held in LDS, at most 4
       case 0:
@@ -1178,6 +1203,15 @@ bool decf_enabled() {
   return on;
 }
 
+// LDS of a k_decode block without its weight words: X, S, red[32], vals[4 parts x 48] (sized for
+// the most parts any kind takes) and the encoded activations.
+size_t dec_lds(DecKind kind, int mode, const Geom& g) {
+  const int Lc = g.Lc, na = kind == kIFG ? 3 : 1;
+  const size_t WL = 8 * static_cast<size_t>((Lc + 31) / 32 * 32 + 4) + 8, LQ = Lc + 16;
+  const size_t lds = (2 * WL + 32 + 4 * 48) * sizeof(float);
+  return lds + (mode == kFloat ? na * WL * sizeof(float) : na * (16 * LQ + 8 * sizeof(int32_t)) + 4 * sizeof(float));
+}
+
 template <int MODE>
 hipError_t dec_mode(DecKind kind, const DecArgs& a, hipStream_t s) {
   if (kind == kOp) return decf_kind<MODE, kOp>(a, s);
@@ -1192,21 +1226,17 @@ hipError_t dec_mode(DecKind kind, const DecArgs& a, hipStream_t s) {
     if (e != hipErrorNotSupported) return e;
   }
   const Geom& g = a.p[0].g;
-  const int Lc = g.Lc;
-  const int na = kind == kIFG ? 3 : 1;
-  const size_t WL = 8 * static_cast<size_t>((Lc + 31) / 32 * 32 + 4) + 8, LQ = Lc + 16;
-  // X, S, red[32], vals[4 parts x 48]: sized for the most parts any kind takes
-  size_t lds = (2 * WL + 32 + 4 * 48) * sizeof(float);
-  lds += (MODE == kFloat) ? na * WL * sizeof(float) : na * (16 * LQ + 8 * sizeof(int32_t)) + 4 * sizeof(float);
+  size_t lds = dec_lds(kind, MODE, g);
   const int nout = (kind == kGate) ? g.N / 2 : g.N;
-  int grid = (nout + kGroup - 1) / kGroup;
-  if (kind == kLM) grid = lm_blocks(grid, g.K);
+  int blocks = (nout + kGroup - 1) / kGroup;
+  if (kind == kLM) blocks = lm_blocks(blocks, g.K);
+  const dim3 grid(blocks, a.streams > 1 ? a.streams : 1);
   // all weight words of the block's output groups go to LDS at entry when they fit (the
   // lm_head's blocks stride over several groups)
   DecArgs b = a;
   b.wgroups = 0;
   const int nm = kind == kIFG ? 3 : (kind == kGate ? 2 : 1);
-  const int G = (kind == kLM) ? (((nout + kGroup - 1) / kGroup) + grid - 1) / grid : 1;
+  const int G = (kind == kLM) ? (((nout + kGroup - 1) / kGroup) + blocks - 1) / blocks : 1;
   const size_t wx = static_cast<size_t>(nm) * G * g.Wc * 128 * sizeof(uint32_t);
   // float layer GEMVs: the fp4 slab (twice the words) when every matrix has one and its words
   // fit in LDS beside the rest; otherwise the 2-bit slab
@@ -1248,7 +1278,28 @@ __global__ void k_to_chain(const float* __restrict__ x, float* __restrict__ out,
   }
 }
 
+// One wave per stream: the token of the stream's per-block lm_head keys.
+__global__ __launch_bounds__(64) void k_argmax_keys(const unsigned long long* __restrict__ keys, int n,
+                                                    int64_t* __restrict__ ids) {
+  const unsigned long long* kb = keys + static_cast<size_t>(blockIdx.x) * kLMBlocks;
+  unsigned long long best = 0ull;
+  for (int e0 = threadIdx.x; e0 < n; e0 += 8 * 64) {
+    unsigned long long k[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) k[u] = e0 + u * 64 < n ? kb[e0 + u * 64] : 0ull;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) best = k[u] > best ? k[u] : best;
+  }
+  best = wave_max_u64(best);
+  if (threadIdx.x == 0) ids[blockIdx.x] = key_index(best);
+}
+
 }  // namespace
+
+hipError_t launch_argmax_keys(const unsigned long long* keys, int n, int streams, int64_t* ids, hipStream_t s) {
+  k_argmax_keys<<<streams, 64, 0, s>>>(keys, n, ids);
+  return hipGetLastError();
+}
 
 hipError_t launch_decode(DecKind kind, Mode mode, const DecArgs& a, hipStream_t s) {
   switch (mode) {
@@ -1256,6 +1307,14 @@ hipError_t launch_decode(DecKind kind, Mode mode, const DecArgs& a, hipStream_t 
     case kFixed: return dec_mode<kFixed>(kind, a, s);
     default: return dec_mode<kInt8>(kind, a, s);
   }
+}
+
+bool decode_fits(DecKind kind, Mode mode, const Geom& g) {
+  // the fewest threads a block of this kind can have (one part of the lm_head, kParts else)
+  const int nm = kind == kIFG ? 3 : (kind == kGate ? 2 : 1);
+  const int ks = (mode == kFloat || kind == kLM) ? 1 : ((kind == kO || kind == kDown) ? 4 : 2);
+  const int F4 = (8 * g.Lc + 8) / 4;
+  return F4 <= 16 * kBlock * nm * ks && dec_lds(kind, mode, g) <= static_cast<size_t>(lds_limit());
 }
 
 hipError_t launch_to_chain(const float* x, float* out, int rows, int K, int Lc, hipStream_t s) {

@@ -122,6 +122,11 @@ struct RowScratch {
   DBuf chunk;  // chunk summaries and starting states of the chunked scan
 };
 
+// Vectors of a fused serving step, one chain-transposed vector per stream (zero padding).
+struct StepScratch {
+  DBuf h, resid, g, recur, z, keys;
+};
+
 struct Model {
   mmf_config cfg{};
   bool begun = false, finalized = false;
@@ -142,6 +147,7 @@ struct Model {
   DBuf state;  // [L][B][H]
   size_t streams = 0;
   RowScratch rs;
+  StepScratch ss;
   // decode graph
   hipGraphExec_t graph = nullptr;
   bool graph_tried = false;
@@ -664,14 +670,21 @@ void lm_single(mmf_ctx* c, Model& m, const float* x, float* logits, bool want_ke
 // layer 0 then gathers the embedding row of the argmax key (recording it in the token
 // history) and its kO clears the key for this step's lm_head. Timing runs use full =
 // false (layer 0 reads h like the others).
-void decode_one(mmf_ctx* c, Model& m, DecKind kind, size_t l, bool full = false) {
+//
+// streams > 0: one kernel of a fused serving step of that many streams instead (blockIdx.y the
+// stream, vectors in m.ss, one step at a time): layer 0 gathers the embedding rows of the
+// device tokens, and the last layer's output goes to hnat [streams][H] in natural order if
+// given.
+void decode_one(mmf_ctx* c, Model& m, DecKind kind, size_t l, bool full = false, size_t streams = 0,
+                const int64_t* tokens = nullptr, float* hnat = nullptr) {
   const Mode mode = static_cast<Mode>(m.mode);
   const size_t H = m.cfg.hidden_size;
-  float* h = static_cast<float*>(m.h.p);
-  float* resid = static_cast<float*>(m.resid.p);
-  float* g = static_cast<float*>(m.g.p);
-  float* recur = static_cast<float*>(m.recur.p);
-  float* z = static_cast<float*>(m.z.p);
+  const bool st = streams > 0;
+  float* h = static_cast<float*>(st ? m.ss.h.p : m.h.p);
+  float* resid = static_cast<float*>(st ? m.ss.resid.p : m.resid.p);
+  float* g = static_cast<float*>(st ? m.ss.g.p : m.g.p);
+  float* recur = static_cast<float*>(st ? m.ss.recur.p : m.recur.p);
+  float* z = static_cast<float*>(st ? m.ss.z.p : m.z.p);
   float* state = static_cast<float*>(m.state.p);
   if (kind == kLM) {
     lm_single(c, m, h, nullptr, true);
@@ -680,19 +693,23 @@ void decode_one(mmf_ctx* c, Model& m, DecKind kind, size_t l, bool full = false)
   const LayerDev& L = m.layers[l];
   DecArgs a = dec_base(m);
   a.layer = static_cast<int>(l);
+  a.streams = static_cast<int>(streams);
+  a.tokens = tokens;
   switch (kind) {
     case kIFG:
       for (int k = 0; k < 3; ++k) set_proj(c, m, a, k, L.proj[k]);
       a.x = (l == 0 && full) ? nullptr : h;
       if (a.x == nullptr) {
         a.out = h;  // layer 0: the embedding row becomes h
-        a.hist = m.hist.as<int64_t>(1);
-        a.hist_pos = m.hist_pos.as<int32_t>(1);
-        a.hist_cap = static_cast<int>(m.hist_cap);
+        if (!st) {
+          a.hist = m.hist.as<int64_t>(1);
+          a.hist_pos = m.hist_pos.as<int32_t>(1);
+          a.hist_cap = static_cast<int>(m.hist_cap);
+        }
       }
       a.pre_w = L.attnT;
       a.lb = L.lb;
-      a.state = state + l * H;
+      a.state = state + l * (st ? streams : 1) * H;
       a.recur = recur;
       a.gout = g;
       break;
@@ -717,6 +734,10 @@ void decode_one(mmf_ctx* c, Model& m, DecKind kind, size_t l, bool full = false)
       a.x = z;
       a.hin = resid;
       a.out = h;
+      if (hnat && l + 1 == m.layers.size()) {
+        a.out = hnat;
+        a.out_nat = 1;
+      }
       break;
   }
   // each fused launch is one BitLinear group (with its norms and epilogue): timed as matmul
@@ -776,6 +797,43 @@ void decode_step(mmf_ctx* c, Model& m) {
   } else {
     decode_launches(c, m);
   }
+}
+
+// The fused serving step's vectors for B streams, zeroed where they grew (their padding stays
+// zero: only valid positions are ever written).
+void alloc_step(mmf_ctx* c, Model& m, size_t B) {
+  StepScratch& s = m.ss;
+  const size_t bH = B * chain_len(m.gH) * sizeof(float), bI = B * chain_len(m.gI) * sizeof(float);
+  for (DBuf* b : {&s.h, &s.resid, &s.g, &s.recur, &s.z}) {
+    const size_t n = b == &s.z ? bI : bH;
+    if (n <= b->n) continue;
+    b->get(n);
+    MMF_HIP(hipMemsetAsync(b->p, 0, n, c->stream));
+  }
+  s.keys.as<unsigned long long>(B * kLMBlocks);
+}
+
+// Most streams whose lm_head runs on the decode kernel, where every block recomputes its stream's
+// final norms; more take the row prologue and GEMM. Measured steps (four layers, vocabulary
+// 32000, float / FixedQ510): 4 streams of the 2.7B width 383 / 396 us against 431 / 425 with the
+// row lm_head; 8 streams of the 370M width 196 / 210 against 175 / 186.
+constexpr size_t kLMFusedMax = 4;
+
+// Whether the serving step of B streams runs on the fused decode kernels: half the row path's
+// launches, but every block recomputes its stream's norms, so their time grows with B times the
+// width while the row path's matrix-core GEMMs (from 8 integer or 16 float rows) hardly grow.
+// Steps of four layers, row path -> fused (us): 1 stream 370M float 213 -> 118, 1.3B FixedQ510
+// 319 -> 161; 8 x 370M FixedQ510 226 -> 186; 4 x 1.3B FixedQ510 649 -> 288, 8 x 308 -> 439;
+// float 16 x 370M 310 -> 235, 8 x 1.3B 517 -> 445, 6 x 2.7B 605 -> 494, 12 x 1.3B 561 -> 592.
+// Several streams need H % 8 == 0, so that no element of the gate math over all B * H elements
+// is a SIMD tail element (the row path's rule). The kernels must fit the widths.
+bool step_fused(const Model& m, size_t B) {
+  const size_t H = m.cfg.hidden_size;
+  const Mode mode = static_cast<Mode>(m.mode);
+  if (m.ext_on() || (B > 1 && (H % 8 != 0 || B * H > (mode == kFloat ? 16384u : 8192u)))) return false;
+  for (DecKind k : {kIFG, kO, kGate, kLM})
+    if (!decode_fits(k, mode, m.gH)) return false;
+  return decode_fits(kDown, mode, m.gI);
 }
 
 void drop_graph(Model& m) {
@@ -1008,6 +1066,8 @@ void mmf_destroy(mmf_ctx* c) {
   for (DBuf* b : {&s.ids, &s.h, &s.resid, &s.i, &s.f, &s.g, &s.recur, &s.scan, &s.z, &s.logits, &s.state0, &s.am,
                   &s.acty, &s.actq, &s.actct, &s.actsa, &s.segs, &s.chunk})
     b->release();
+  StepScratch& ss = m.ss;
+  for (DBuf* b : {&ss.h, &ss.resid, &ss.g, &ss.recur, &ss.z, &ss.keys}) b->release();
   for (DBuf* b : {&c->raw, &c->opy, &c->opq, &c->opct, &c->opsa, &c->opstate, &c->gws, &c->hmx, &c->hmacc})
     b->release();
   c->pin_x.release();
@@ -1716,8 +1776,33 @@ namespace {
 
 // The launches of one lockstep serving step of the m.streams streams: embedding of the
 // device tokens d, every layer over the B rows, final norm + lm_head into lg, argmax into am.
+// Few streams (step_fused) run the fused decode kernels, four launches per layer over a grid of
+// (blocks, streams); the lm_head of one stream is the decode kernel's, of several the row one.
 void step_kernels(mmf_ctx* c, Model& m, const int64_t* d, float* h, float* lg, int64_t* am) {
   const size_t B = m.streams, H = m.cfg.hidden_size, V = m.cfg.vocab_size;
+  if (step_fused(m, B)) {
+    for (size_t l = 0; l < m.layers.size(); ++l)
+      for (DecKind k : {kIFG, kO, kGate, kDown}) decode_one(c, m, k, l, true, B, d, B > kLMFusedMax ? h : nullptr);
+    if (B <= kLMFusedMax) {
+      DecArgs a = dec_base(m);
+      set_proj(c, m, a, 0, m.lm);
+      a.x = static_cast<const float*>(m.ss.h.p);
+      a.pre_w = m.norm_wT;
+      a.out = lg;
+      a.keys = static_cast<unsigned long long*>(m.ss.keys.p);
+      a.streams = static_cast<int>(B);
+      tbeg(c, kRkLM);
+      MMF_HIP(launch_decode(kLM, static_cast<Mode>(m.mode), a, c->stream));
+      MMF_HIP(launch_argmax_keys(a.keys, a.nkeys, static_cast<int>(B), am, c->stream));
+      tend(c);
+      return;
+    }
+    lm_rows(c, m, static_cast<int>(B), h, lg);
+    tbeg(c, kRkLM);
+    MMF_HIP(launch_argmax_rows(lg, static_cast<int>(B), static_cast<int>(V), am, c->stream));
+    tend(c);
+    return;
+  }
   tbeg(c, kRkOther);
   MMF_HIP(launch_embed(m.emb, d, h, static_cast<int>(B), static_cast<int>(H), c->stream));
   tend(c);
@@ -1746,6 +1831,7 @@ int mmf_model_step(mmf_ctx* c, const int64_t* tokens, float* logits, int64_t* ar
     float* h = s.h.as<float>(B * H);
     float* lg = s.logits.as<float>(B * V);
     int64_t* am = s.am.as<int64_t>(B);
+    if (step_fused(m, B)) alloc_step(c, m, B);
     // embedding, all layers, final norm + lm_head, argmax: captured once per stream count
     // and replayed while no scratch buffer has moved (the first step runs them directly)
     auto work = [&] { step_kernels(c, m, d, h, lg, am); };
@@ -1995,6 +2081,7 @@ int mmf_model_time_step(mmf_ctx* c, const int64_t* tokens, int warmup, int reps,
     float* h = s.h.as<float>(B * H);
     float* lg = s.logits.as<float>(B * V);
     int64_t* am = s.am.as<int64_t>(B);
+    if (step_fused(m, B)) alloc_step(c, m, B);
     auto f = [&] { step_kernels(c, m, d, h, lg, am); };
     for (int i = 0; i < warmup; ++i) f();
     time_kinds(c, reps, f, kind_us);

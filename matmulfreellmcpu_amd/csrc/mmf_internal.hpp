@@ -92,6 +92,12 @@ struct DecArgs {
                           // are copied into LDS at entry (0: read from global in the GEMV)
   int32_t* acc;           // kOp, integer modes: the int32 accumulators [N] (tails and the
                           // Q5.10 bias included), or null
+  // A serving step of `streams` independent streams (0 or 1: one): blockIdx.y is the stream.
+  // Every vector above is then an array of streams, 8*Lc + 8 floats apart (state: H apart,
+  // logits: vocab apart, keys: kLMBlocks apart).
+  int streams;
+  const int64_t* tokens;  // kIFG layer 0: the streams' tokens (in [0, vocab)), or null: *key
+  int out_nat;            // kDown: out is [streams][N] in natural order (the row lm_head's input)
 };
 
 // Bytes of dynamic LDS one block may allocate on the current device.
@@ -106,6 +112,9 @@ inline int lm_blocks(int groups, int K) {
   return groups < cap ? groups : cap;
 }
 hipError_t launch_decode(DecKind kind, Mode mode, const DecArgs& a, hipStream_t s);
+// Whether launch_decode has a launch for this kind over geometry g (rows that fit the block
+// layout and LDS).
+bool decode_fits(DecKind kind, Mode mode, const Geom& g);
 // Timing runs: while both events are set, launch_decode records them at its kernel's own start
 // and end (hipExtLaunchKernelGGL), the timestamps a profiler's kernel trace reports, instead of
 // around the launch on the stream.
@@ -283,6 +292,8 @@ hipError_t launch_rmsnorm(const float* x, const float* w, float* y, int rows, in
 hipError_t launch_quant_rows(const float* y, int32_t* q, int rows, int K, float qs, hipStream_t s);
 // Row argmax over [rows, V] logits -> ids.
 hipError_t launch_argmax_rows(const float* logits, int rows, int V, int64_t* ids, hipStream_t s);
+// ids[b] = the index of the largest of stream b's n argmax keys (kLMBlocks apart).
+hipError_t launch_argmax_keys(const unsigned long long* keys, int n, int streams, int64_t* ids, hipStream_t s);
 // Elementwise ops for the op-level API (kernels.hpp:54-68).
 hipError_t launch_swiglu(const float* a, const float* b, float* out, size_t n, hipStream_t s);
 hipError_t launch_swishgate(const float* g, const float* o, const float* w, float* out, int rows,
