@@ -474,7 +474,7 @@ void layer_rows(mmf_ctx* c, Model& m, int l, int rows, float* h, float* state, b
   }
   // gate, lower bound, swiglu, recurrence (hgrn_model.cpp:109-150). Independent streams
   // without a trace: the step runs inside the g_norm prologue below (kPreMixSwish), which
-  // reports hipErrorNotSupported, launching nothing, where its float4 form does not apply.
+  // reports hipErrorNotSupported, launching nothing, where its rows are too long.
   const bool mix_in_prologue = stream_state && !segs && !trace_dev;
   auto run_mixer = [&]() -> hipError_t {
     tbeg(c, kRkMixer);

@@ -183,8 +183,8 @@ struct PrologueArgs {
   float* mix_state;    // kPreMixSwish: recurrent state [rows, K], read and updated
   const float* mix_lb; // kPreMixSwish: lower bounds [K] or null
 };
-// kPreMixSwish runs only in the float4 prologue: it returns hipErrorNotSupported, launching
-// nothing, where that does not apply (the caller then runs launch_mixer and kPreSwish).
+// kPreMixSwish runs only in k_rowpro's forms: it returns hipErrorNotSupported, launching
+// nothing, where rows are too long for them (the caller then runs launch_mixer and kPreSwish).
 hipError_t launch_prologue(Mode mode, const PrologueArgs& a, ActBuf& act, hipStream_t s);
 
 // Integer codes [rows, K] (int16-range, as int32) -> planes (TernaryBackend path).

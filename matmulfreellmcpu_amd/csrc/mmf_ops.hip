@@ -373,6 +373,9 @@ __global__ void k_prologue(PrologueArgs a, ActBuf act) {
   }
 }
 
+// four floats at any 4-byte address (one 16-byte global load or store)
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+
 __device__ __forceinline__ float f4el(const float4& f, int c) {
   return c == 0 ? f.x : (c == 1 ? f.y : (c == 2 ? f.z : f.w));
 }
@@ -390,11 +393,12 @@ constexpr int rowpro_waves() {
   return (BT == 256 && entry <= 24 && encode <= 40) ? 8 : 1;
 }
 
-// The row prologue for K % 4 == 0 with 16-byte aligned inputs and the chain-transposed norm
-// weights normwT. One block per row; each thread owns
+// The row prologue with the chain-transposed norm weights normwT. One block per row; each thread
+// owns
 //  - groups (the loads and the element-wise stage 1): group t < G = nb + (ntail > 0) is the
-//    eight elements 8t .. 8t+7, chain position t of every chain (two float4 loads), or for
-//    t = nb the ntail (= 4) tail elements. Its values go to the chain-transposed LDS row
+//    eight elements 8t .. 8t+7, chain position t of every chain (two 16-byte loads, which
+//    global memory takes at any 4-byte alignment, so K and the row addresses are free), or for
+//    t = nb the ntail tail elements (one by one). Its values go to the chain-transposed LDS row
 //    X[c * LS + t] (tail: X[8 * LS + c]) that the order-fixed norm chains read;
 //  - units (the BitLinear norm and the encoding): unit u < Lc is positions t0 .. t0+7 of
 //    chain j (u = j * Lc/8 + t0/8). Its eight normed values come from two LDS reads and two
@@ -404,7 +408,9 @@ constexpr int rowpro_waves() {
 // memory round trip); the BitLinear norm weights of the thread's units are loaded before the
 // second norm chain (projection 0) or while the previous projection is encoded, so their
 // latency hides behind work -- or, with PW (a few rows per launch: a launch is one row's
-// latency), at entry too. Arithmetic and order are those of k_prologue.
+// latency), at entry too. Arithmetic and order are those of k_prologue, which widths that are no
+// multiple of 4 and unaligned rows took before (Int8Absmax, us per launch: 100 x 1031 8 -> 7,
+// 300 x 6911 20 -> 13, 1111 x 6911 48 -> 17) and rows too long for a thread's units still do.
 template <int MODE, int PRE, int NA, int MAXG, bool PW, int BT>
 __global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(rowpro_waves<MODE, PRE, NA, MAXG, BT>())))
 void k_rowpro(PrologueArgs a, ActBuf act) {
@@ -429,14 +435,22 @@ void k_rowpro(PrologueArgs a, ActBuf act) {
     j = static_cast<int>(__umulhi(static_cast<uint32_t>(u), mL8));
     t0 = 8 * (u - j * L8);
   };
-  // elements 8t .. 8t+7 of a K-long vector: two float4, or for the tail group one and zeros
-  // (the tail group's second load repeats its first, an address in bounds, and is replaced by
-  // zeros: a select of values, not of addresses)
+  // elements 8t .. 8t+7 of a K-long vector, or for the tail group its ntail and zeros
   auto ld8 = [&](const float* p, int t, float4* o) {
-    const float4* p4 = reinterpret_cast<const float4*>(p) + 2 * t;
-    const float4 h = p4[t < nb ? 1 : 0];
-    o[0] = p4[0];
-    o[1] = t < nb ? h : z4;
+    if (t < nb) {
+      const f4u* p4 = reinterpret_cast<const f4u*>(p + 8 * t);
+      const f4u l = p4[0], h = p4[1];
+      o[0] = make_float4(l.x, l.y, l.z, l.w);
+      o[1] = make_float4(h.x, h.y, h.z, h.w);
+    } else {
+      float e[8];
+#pragma unroll
+      for (int c = 0; c < 8; ++c) e[c] = p[K8 + (c < nt ? c : 0)];
+#pragma unroll
+      for (int c = 0; c < 8; ++c) e[c] = c < nt ? e[c] : 0.0f;
+      o[0] = make_float4(e[0], e[1], e[2], e[3]);
+      o[1] = make_float4(e[4], e[5], e[6], e[7]);
+    }
   };
   const size_t rK = static_cast<size_t>(row) * K;
 
@@ -499,9 +513,15 @@ void k_rowpro(PrologueArgs a, ActBuf act) {
         const float in = swiglu_of(x2s[c], 1.0f - f, tail);
         st[c] = __builtin_fmaf(f, f4el(sv[g][c >> 2], c & 3), in);
       }
-      float4* so = reinterpret_cast<float4*>(a.mix_state + rK) + 2 * t;
-      so[0] = make_float4(st[0], st[1], st[2], st[3]);
-      if (t < nb) so[1] = make_float4(st[4], st[5], st[6], st[7]);
+      float* so = a.mix_state + rK + 8 * t;
+      if (t < nb) {
+        reinterpret_cast<f4u*>(so)[0] = f4u{st[0], st[1], st[2], st[3]};
+        reinterpret_cast<f4u*>(so)[1] = f4u{st[4], st[5], st[6], st[7]};
+      } else {
+#pragma unroll
+        for (int c = 0; c < 7; ++c)
+          if (c < nt) so[c] = st[c];
+      }
 #pragma unroll
       for (int c = 0; c < 8; ++c) x2s[c] = st[c];
     }
@@ -2042,14 +2062,19 @@ static hipError_t rowseg_launch(const PrologueArgs& a, ActBuf& act, hipStream_t 
 
 template <int MODE, int PRE, int NA>
 static hipError_t rowpro_inst(const PrologueArgs& a, ActBuf& act, size_t lds, hipStream_t s) {
-  if (rowseg_enabled()) {
+  // the segment and half-row kernels load aligned float4
+  bool al = act.K % 4 == 0 && aligned16(a.x);
+  if (PRE != kPreNone) al = al && aligned16(a.pre_w);
+  if (PRE == kPreSwish || PRE == kPreMixSwish) al = al && aligned16(a.x2);
+  if (PRE == kPreMixSwish) al = al && aligned16(a.mix_f) && aligned16(a.mix_state) && (!a.mix_lb || aligned16(a.mix_lb));
+  if (al && rowseg_enabled()) {
     const hipError_t e = rowseg_launch<MODE, PRE, NA>(a, act, s);
     if (e != hipErrorNotSupported) return e;
   }
   const int need = rowpro_need(act), grid = row_grid(act.rows);
   if constexpr (PRE == kPreNone && NA == 1 && MODE != kInt8) {
     // long rows of many-row launches: half of the row in LDS at a time (k_rowpro_split)
-    if (act.rows > kPrologueFewRows && need > 512 && need <= 1024 && act.nb >= 512 && aligned16(a.normw[0])) {
+    if (al && act.rows > kPrologueFewRows && need > 512 && need <= 1024 && act.nb >= 512 && aligned16(a.normw[0])) {
       const size_t lds_split = (8 * static_cast<size_t>(host_lds_stride(std::max(512, act.Lc - 512))) + 8 + 32) * sizeof(float);
       if (need <= 768) k_rowpro_split<MODE, 3><<<grid, 256, lds_split, s>>>(a, act);
       else k_rowpro_split<MODE, 4><<<grid, 256, lds_split, s>>>(a, act);
@@ -2087,14 +2112,9 @@ hipError_t launch_prologue(Mode mode, const PrologueArgs& a, ActBuf& act, hipStr
   const size_t lds = (2 * rowf + 16) * sizeof(float);
   const bool sw = a.pre == kPreSwish || a.pre == kPreMixSwish;
   const size_t lds4 = ((sw ? 2 : 1) * rowf + 32) * sizeof(float);  // k_rowpro
-  bool fast = act.K % 4 == 0 && rowpro_fits(act) && aligned16(a.x) && (a.na == 1 || a.na == 3);
-  if (a.pre != kPreNone) fast = fast && aligned16(a.pre_w);
-  if (sw) fast = fast && aligned16(a.x2);
+  bool fast = rowpro_fits(act) && (a.na == 1 || a.na == 3);
   for (int i = 0; i < a.na; ++i) fast = fast && a.normwT[i] && aligned16(a.normwT[i]);
-  if (a.pre == kPreMixSwish) {
-    fast = fast && a.na == 1 && aligned16(a.mix_f) && aligned16(a.mix_state) && (!a.mix_lb || aligned16(a.mix_lb));
-    if (!fast) return hipErrorNotSupported;
-  }
+  if (a.pre == kPreMixSwish && !(fast && a.na == 1)) return hipErrorNotSupported;
   if (fast) {
     hipError_t e = hipErrorNotSupported;
     switch (mode) {

@@ -1,0 +1,69 @@
+"""BitLinear at widths and row addresses that fit no vector load or tile, against the CPU
+restatement, bit for bit: the float4-free row prologue, the tail terms and the partial tiles of
+the integer matrix-core epilogues."""
+import numpy as np
+import pytest
+
+from conftest import assert_bitexact
+from test_gpu_parity import Dev, eng  # noqa: F401  (module fixture)
+
+pytestmark = pytest.mark.gpu
+
+FLOAT, FIXED, INT8 = 0, 1, 2
+
+# (rows, K, N): K % 8 from 0 to 7, one and two units per thread of the few-row prologue, one to
+# four of the many-row one, rows below, at and above a row tile
+SHAPES = [(2, 9, 33), (3, 1025, 70), (5, 4098, 64), (8, 1031, 130), (13, 516, 95), (31, 2047, 1333), (33, 130, 6000),
+          (48, 1030, 200), (64, 300, 2100), (65, 1027, 64), (100, 1031, 1333), (130, 8190, 40), (300, 255, 500),
+          (520, 1029, 36), (530, 2046, 36), (515, 4099, 36), (514, 6911, 36), (513, 8187, 36), (514, 5632, 36)]
+
+
+@pytest.mark.parametrize("mode", [FLOAT, FIXED, INT8])
+@pytest.mark.parametrize("rows,K,N", SHAPES)
+def test_bitlinear_odd(eng, oracle, rows, K, N, mode):  # noqa: F811
+    print(f"odd rows={rows} K={K} N={N} mode={mode}", flush=True)
+    rng = np.random.default_rng(rows + 3 * K + 5 * N + mode)
+    x = (rng.standard_normal((rows, K)) * 2).astype(np.float32)
+    nw = (1 + 0.1 * rng.standard_normal(K)).astype(np.float32)
+    wq = rng.integers(-1, 2, (N, K)).astype(np.int8)
+    sw = float(np.float32(1.0 / 0.0157))
+    want = oracle.bitlinear(x, nw, wq, sw, 1e-6, mode)
+    pid = eng.register_proj(wq, sw, nw)
+    for off in (0, 1):  # the rows one float past an aligned address
+        buf = np.zeros(rows * K + off, np.float32)
+        buf[off:] = x.ravel()
+        dx, dout = Dev(eng, buf), Dev(eng, shape=(rows, N))
+        dacc = Dev(eng, shape=(rows, N), dtype=np.int32)
+        for acc in ((None,) if mode == FLOAT else (dacc.ptr, None)):
+            eng.bitlinear(pid, dx.ptr + 4 * off, dout.ptr, rows, mode=mode, acc=acc)
+            eng.sync()
+            assert_bitexact(dout.get(), want["out"], f"out offset {off}")
+        if mode != FLOAT:
+            np.testing.assert_array_equal(dacc.get(), want["acc"])
+    eng.proj_release(pid)
+
+
+@pytest.mark.parametrize("hidden", [100, 250, 1027])
+@pytest.mark.parametrize("mode", [FLOAT, FIXED, INT8])
+def test_serve_odd_hidden(tmp_path, oracle, hidden, mode):
+    """Serving steps whose recurrence runs inside the g_norm prologue at hidden sizes that are no
+    multiple of 4 (rows at any 4-byte address, one to seven tail elements)."""
+    from matmulfreellmcpu_amd import Engine, make_blob, read_blob
+    print(f"serve hidden={hidden} mode={mode}", flush=True)
+    blob = read_blob(make_blob(str(tmp_path / "m"), vocab=500, hidden=hidden, layers=2, inter=208, seed=hidden,
+                               random_norms=True, random_lb=True))
+    om = oracle.model(blob)
+    rng = np.random.default_rng(hidden + mode)
+    prompts = [rng.integers(0, 500, n) for n in (5, 9, 1, 20, 3)]
+    want, wst = om.generate_serve(prompts, 4, mode, want_state=True)
+    e = Engine(0)
+    e.load_blob(blob, mode)
+    e.reset(len(prompts))
+    got = [list(p) + [int(t)] for p, t in zip(prompts, e.prefill_streams(prompts))]
+    for _ in range(3):
+        for g, t in zip(got, e.step([g[-1] for g in got])):
+            g.append(int(t))
+    for g, w in zip(got, want):
+        np.testing.assert_array_equal(np.array(g), w)
+    assert_bitexact(e.state(), wst, "states")
+    e.close()
