@@ -215,8 +215,8 @@ struct GemmArgs {
   // Q5.10 bias included, as an external integer matmul returns them)
   bool ext_acc;
 };
-// Dispatches the integer modes to the matrix-core kernel (mmf_mfma.hip) from
-// mfma_min_rows() rows on, everything else to the dot-product kernel.
+// Dispatches the integer modes to the matrix-core kernel (mmf_mfma.hip) where
+// int_mfma_rows(), everything else to the dot-product kernel.
 hipError_t launch_gemm(const GemmArgs& a, const ActBuf& act, hipStream_t s);
 hipError_t launch_gemm_mfma(const GemmArgs& a, const ActBuf& act, hipStream_t s);
 // Dequantisation and output stage (a.epi) of complete integer accumulators a.ws
@@ -250,9 +250,12 @@ hipError_t measure_peaks(int cus, hipStream_t s, double out[4]);
 // Bytes of int32 workspace launch_gemm needs for `a` (0 when it will not split K); the
 // caller passes at least that much in a.ws.
 size_t gemm_workspace_bytes(const GemmArgs& a);
-// Rows from which the integer modes use the matrix cores (MMF_MFMA_MIN_ROWS, default 8;
-// 0 disables them).
-int mfma_min_rows();
+// Whether the integer modes run a GEMM of these rows over K on the matrix cores: from 3 (FixedQ510)
+// or 4 rows, and below where rows * K >= 1024 (us per BitLinear call, dot products -> matrix
+// cores: 2 x 1024 x 5632 FixedQ510 11.3 -> 7.1, Int8Absmax 8.2 -> 7.1, 7 rows 21.8 -> 7.3, 3 x 64 x
+// 64 FixedQ510 6.5 -> 6.3; but 3 x 64 x 3000 Int8Absmax 6.9 -> 7.5, 2 x 300 x 6000 8.5 -> 9.1).
+// MMF_MFMA_MIN_ROWS sets another row count (0: never).
+bool int_mfma_rows(Mode mode, int rows, int K);
 // Rows from which float mode uses the fp32 matrix cores (MMF_FLOAT_MFMA_MIN_ROWS, default
 // 16; 0 disables them).
 int float_mfma_min_rows();

@@ -36,15 +36,15 @@
 // stages ahead, this measured 10% faster on the long-prefill shapes; most of the remaining
 // gap to the matrix-core peak is the stage barriers' LDS-read bubble, the output stores
 // after the loop, and whole-chip rounds of tiles.)
-// Split-K: when a GEMM has too few tiles to occupy the chip (a few dozen rows, or narrow
-// matrices), blockIdx.y selects a contiguous range of stages; each block stores its exact
-// int32 partial tile, and k_splitk_epi adds the partials in split order and applies the
-// epilogue (integer sums: the order does not change the result).
-//
-// K-groups (KW > 1): the split can also live inside one block. Its waves form KW groups of
-// WM x WN waves that take equal runs of the stages of the same tile, each through its own
-// LDS slots; group 0 adds the others' int32 tiles from LDS and runs the epilogue. That
-// gives more waves per SIMD (or no partials through memory) with the same tile traffic.
+// K-groups (KW > 1): the stages of one tile can be split inside one block. Its waves form KW
+// groups of WM x WN waves that take equal runs of the stages, each through its own LDS slots;
+// their int32 tiles meet in LDS and the waves share the sum and the epilogue. That gives more
+// waves per SIMD with the same tile traffic and no partials through memory: eight one-wave
+// groups carry every launch of up to a few hundred small tiles, two groups the 128 x 128 tiles
+// at one block per CU.
+// Split-K (K beyond 6912 with few tiles): blockIdx.y selects a contiguous range of stages; each
+// block stores its exact int32 partial tile, and k_splitk_epi adds the partials in split order
+// and applies the epilogue (integer sums: the order does not change the result).
 #include <cstdlib>
 #include <type_traits>
 
@@ -143,10 +143,11 @@ template <int MODE, int WM, int WN, int FM, int FN, int KQ>
 __host__ __device__ constexpr int stage_bytes() {
   return ((MODE == kFixed) ? 2 : 1) * FM * WM * KQ * 1024 + FN * WN * KQ * 256;
 }
-// LDS bytes of a block beside its stage ring: the int8 row divisors and their reciprocals.
+// LDS bytes of a block beside its stage ring: the int8 row divisors and their reciprocals, and
+// the rows' eight tail codes.
 template <int MODE, int WM, int FM>
 __host__ __device__ constexpr int row_scale_bytes() {
-  return (MODE == kInt8 ? 2 : 1) * 32 * FM * WM * 4;
+  return ((MODE == kInt8 ? 2 : 1) + 8) * 32 * FM * WM * 4;
 }
 // Depth of the stage ring: as many slots (at most 6) as fit the LDS of the blocks a CU
 // holds (two for blocks of at most four waves, else one), with the int8 row scales.
@@ -271,6 +272,7 @@ __global__ __launch_bounds__(64 * WM * WN * KW, (mfma_min_waves<MODE, EPI, WM, W
   }
   const int Nout = (EPI == kEpiSwigluPair) ? N / 2 : N;
   const int ol = lane & 31;
+  constexpr bool PAIR = EPI == kEpiSwigluPair;
   // column (in N) of each of the wave's groups; a swiglu pair's gate group is even and its
   // up partner follows it: gate column (cg/2)*32 + ol, up column Nout + the same
   int col[FN];
@@ -294,9 +296,7 @@ __global__ __launch_bounds__(64 * WM * WN * KW, (mfma_min_waves<MODE, EPI, WM, W
 #pragma unroll
       for (int bj = 0; bj < FN; ++bj) acc[pl][ai][bj] = v16i{};
 
-  // The stage ring: D slots, each its own LDS array (so that the compiler tells the slot
-  // being filled from the slot being read and waits for nothing it need not), each holding
-  // one stage of every K-group ([KW][SS] bytes). Every wave moves its share of a stage (DA
+  // The stage ring: D slots, each holding one stage of every K-group ([KW][SS] bytes). Every wave moves its share of a stage (DA
   // activation transfers of 1 KB, DB weight transfers of 256 B) from global memory straight
   // into a slot with buffer loads into LDS (lds_dma16/4: lane l's bytes land at the
   // transfer's base + l * size), D - 1 stages ahead: no registers and no LDS stores on the
@@ -312,20 +312,15 @@ __global__ __launch_bounds__(64 * WM * WN * KW, (mfma_min_waves<MODE, EPI, WM, W
   constexpr int QB = KW * SS;
   // two-group split of the sum and the epilogue (see after the main loop): each group's four
   // waves send one fragment pair (FN x 4 KB) through two ring slots
-  constexpr bool KW2S = KW == 2 && FM == 2 && NW == 4 && D >= 4 && 2 * FN * 4096 <= QB;
-  __shared__ __align__(16) unsigned char q0[QB], q1[QB], q2[QB], q3[D > 3 ? QB : 16], q4[D > 4 ? QB : 16],
-      q5[D > 5 ? QB : 16];
+  constexpr bool KW2S = KW == 2;
+  static_assert(KW != 2 || (FM == 2 && NW == 4 && D >= 4 && 2 * FN * 4096 <= QB), "the exchange fits the ring");
+  constexpr int GR = FM * FN * 4096;  // bytes of one K-group's fragments (after the loop)
+  constexpr int RB = (KW == 8 && 8 * GR > D * QB) ? 8 * GR : D * QB;
+  __shared__ __align__(16) unsigned char ring[RB];
   __shared__ float srow[BM];  // Int8: the divisor of each row, scale_w * scale_a
   __shared__ float srcp[MODE == kInt8 ? BM : 1];  // Int8: its correctly rounded reciprocal
-  auto slot = [&](auto sc) -> unsigned char* {
-    constexpr int S = decltype(sc)::value;
-    if constexpr (S == 0) return q0;
-    else if constexpr (S == 1) return q1;
-    else if constexpr (S == 2) return q2;
-    else if constexpr (S == 3) return q3;
-    else if constexpr (S == 4) return q4;
-    else return q5;
-  };
+  __shared__ int4 stct[2 * BM];  // the rows' tail codes (K % 8 != 0)
+  auto slot = [&](auto sc) -> unsigned char* { return ring + decltype(sc)::value * QB; };
   auto issue = [&](auto sc, int s2) {
     unsigned char* sb = slot(sc) + kg * SS;
     const int sg = st0 + min(gb + s2, nst - 1);
@@ -433,243 +428,228 @@ __global__ __launch_bounds__(64 * WM * WN * KW, (mfma_min_waves<MODE, EPI, WM, W
     }
     rcp_ok = __syncthreads_and(ok) && act.K < 16384;
   }
-  if constexpr (KW > 1) {
-    // K-group reduction: FixedQ510 folds its planes first (hi * 256 + lo into plane 1, as
-    // the split-K partials do); then in each round groups 1..KW-1 store as many fragments as
-    // a ring slot holds (all of them for the FixedQ510 few-row tiles), group r into slot
-    // r - 1 (free once every wave has passed the barrier that precedes the stores), and after
-    // one more barrier group 0 adds them: 16 bytes per lane per access
+  // The K % 8 tail terms: the rows' codes in LDS, a lane's columns' weights in registers. Codes of 16 bits or less multiply at the 24-bit rate; a wider one (the
+  // Q5.10 code of a NaN) makes the block use 32-bit products.
+  bool wide = false;
+  if (ntail) {
+    bool big = false;
+    if (tid < 2 * BM) {
+      int row = row0 + (tid >> 1);
+      row = row < arows ? row : arows - 1;
+      const int4 c = reinterpret_cast<const int4*>(act_ct + (static_cast<size_t>(am) * arows + row) * 8)[tid & 1];
+      stct[tid] = c;
+      auto w = [](int v) { return v < -32768 || v > 32767; };
+      big = w(c.x) || w(c.y) || w(c.z) || w(c.w);
+    }
+    wide = __syncthreads_or(big);
+  }
+  // the tail weights of column c, two signed bits each (0 without a tail)
+  auto tail_of = [&](int c) {
+    uint32_t t = 0;
+    if (ntail) {
+      const uint2 b = *reinterpret_cast<const uint2*>(tailp + 8 * static_cast<size_t>(c < N ? c : N - 1));
+#pragma unroll
+      for (int k = 0; k < 7; ++k) t |= (((k < 4 ? b.x : b.y) >> (8 * (k & 3))) & 3u) << (2 * k);
+    }
+    return t;
+  };
+  // the tail term of a row's codes and a column's weights
+  auto tail_term = [&](const int4& c0, const int4& c1, uint32_t t) {
+    const int32_t c[7] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z};
+    int32_t sum = 0;
+#pragma unroll
+    for (int k = 0; k < 7; ++k) {
+      const int32_t w = static_cast<int32_t>(t << (30 - 2 * k)) >> 30;
+      sum += wide ? w * c[k] : __mul24(w, c[k]);
+    }
+    return sum;
+  };
+  if constexpr (KW > 1 && MODE == kFixed) {  // fold the planes first (hi * 256 + lo into plane 1)
+#pragma unroll
+    for (int ai = 0; ai < FM; ++ai)
+#pragma unroll
+      for (int bj = 0; bj < FN; ++bj)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          acc[1][ai][bj][i] = acc[0][ai][bj][i] * 256 + acc[1][ai][bj][i];
+          acc[0][ai][bj][i] = 0;
+        }
+  }
+  // Eight one-wave groups: the sums and the epilogue are shared. Every group stores its
+  // fragments; then group g < 4 FM adds row quad g % 4 of row
+  // fragment g / 4 (both column groups) over all eight groups and runs the epilogue for those
+  // rows -- up to eight waves instead of one reading and storing.
+  if constexpr (KW == 8) {
+    static_assert(NW == 1 && FN == 2 && FM <= 2, "one wave per group");
+    auto grp = [&](int g) { return reinterpret_cast<v4i*>(ring + g * GR); };  // [fragment][quad][lane] as int4
+    __syncthreads();
+    {
+      v4i* my = grp(kg);
+#pragma unroll
+      for (int f = 0; f < FM * FN; ++f)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const v16i& v = acc[P - 1][f / FN][f % FN];
+          my[(f * 4 + q) * 64 + lane] = v4i{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+        }
+    }
+    __syncthreads();
+    const int ai = kg >> 2, q = kg & 3;
+    // 32-row tiles: four row quads, four waves; row quads past the last row: none
+    if (kg >= FM * 4 || row0 + ai * 32 + 8 * q >= arows) return;
+    // rows rb + e of this quad (fragment row 8 q + 4 (lane / 32) + e), columns col[bj]
+    const int rb = row0 + ai * 32 + 4 * (lane >> 5) + 8 * q;
+    float res[4][FN];
+    if constexpr (EPI == kEpiAdd) {  // the residuals, all loaded before any is used
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int bj = 0; bj < FN; ++bj)
+          res[e][bj] =
+              addp[static_cast<size_t>(rb + e < arows ? rb + e : arows - 1) * N + (col[bj] < N ? col[bj] : N - 1)];
+    }
+    v4i tot[FN];
+#pragma unroll
+    for (int bj = 0; bj < FN; ++bj) tot[bj] = v4i{0, 0, 0, 0};
+#pragma unroll
+    for (int g = 0; g < 8; ++g) {
+      const v4i* src = grp(g);
+#pragma unroll
+      for (int bj = 0; bj < FN; ++bj) tot[bj] = tot[bj] + src[((ai * FN + bj) * 4 + q) * 64 + lane];
+    }
+    int32_t sacc[4][FN];
+    float val[4][FN];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int bj = 0; bj < FN; ++bj) sacc[e][bj] = tot[bj][e] + csum[bj];
+    if (ntail) {
+      uint32_t tw[FN];
+#pragma unroll
+      for (int bj = 0; bj < FN; ++bj) tw[bj] = tail_of(col[bj]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int rl = rb + e - row0;
+        const int4 c0 = stct[2 * rl], c1 = stct[2 * rl + 1];
+#pragma unroll
+        for (int bj = 0; bj < FN; ++bj) sacc[e][bj] += tail_term(c0, c1, tw[bj]);
+      }
+    }
     if constexpr (MODE == kFixed) {
 #pragma unroll
-      for (int ai = 0; ai < FM; ++ai)
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int bj = 0; bj < FN; ++bj) val[e][bj] = static_cast<float>(sacc[e][bj]) * invf;
+    } else if (rcp_ok) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int bj = 0; bj < FN; ++bj)
+          val[e][bj] = div_by_recip(static_cast<float>(sacc[e][bj]), srow[rb + e - row0], srcp[rb + e - row0]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int bj = 0; bj < FN; ++bj) val[e][bj] = static_cast<float>(sacc[e][bj]) / srow[rb + e - row0];
+    }
+    auto store = [&](auto whole) {  // whole tiles without accumulators: straight stores
+      constexpr bool W = decltype(whole)::value;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (!W && rb + e >= arows) continue;
+        const size_t grow = static_cast<size_t>(rb + e);
+        if constexpr (PAIR) {
+          if (!W && col[0] >= Nout) continue;
+          if (!W && accz) {
+            accz[grow * N + col[0]] = sacc[e][0];
+            accz[grow * N + col[1]] = sacc[e][1];
+          }
+          const size_t o = grow * Nout + col[0];
+          if (W || !rawacc)
+            outz[o] = swiglu_of(val[e][0], val[e][1], !W && static_cast<int64_t>(o) >= (swn & ~7));
+        } else {
+#pragma unroll
+          for (int bj = 0; bj < FN; ++bj) {
+            if (!W && col[bj] >= N) continue;
+            const size_t o = grow * N + col[bj];
+            if (!W && accz) accz[o] = sacc[e][bj];
+            if (W || !rawacc) outz[o] = (EPI == kEpiAdd) ? res[e][bj] + val[e][bj] : val[e][bj];
+          }
+        }
+      }
+    };
+    if (row0 + BM <= arows && (cgb + BG) * 32 <= N && !accz && !rawacc &&
+        (!PAIR || static_cast<size_t>(row0 + BM) * Nout <= static_cast<size_t>(swn & ~7)))
+      store(std::true_type{});
+    else
+      store(std::false_type{});
+    return;
+  }
+  // Two K-groups of two row fragments each (the long-prefill 128 x 128 tiles): the groups
+  // split the sum and the epilogue by row fragment. Group g keeps fragment g, sends its
+  // fragment 1 - g to the same wave of the other group through LDS and adds the one it
+  // receives (exact int32 sums: any order), then stores its own 32-row half of the tile.
+  if constexpr (KW2S) {
+    // (kept and sent fragments as compile-time indices: a run-time index into the
+    // accumulator array would put it in scratch memory)
+    constexpr int XW = FN * 4 * 64;  // int4 of one wave's sent fragment
+    auto exch = [&](auto keepc) {
+      constexpr int KEEP = decltype(keepc)::value, SEND = 1 - KEEP;
+      __syncthreads();
+      {
+        v4i* out = reinterpret_cast<v4i*>(ring) + (KEEP * 4 + wave) * XW;
 #pragma unroll
         for (int bj = 0; bj < FN; ++bj)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            acc[1][ai][bj][i] = acc[0][ai][bj][i] * 256 + acc[1][ai][bj][i];
-            acc[0][ai][bj][i] = 0;
+          for (int q = 0; q < 4; ++q) {
+            const v16i& v = acc[P - 1][SEND][bj];
+            out[(bj * 4 + q) * 64 + lane] = v4i{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
           }
-    }
-    // Eight one-wave groups on a whole in-range tile: the sums and the epilogue are shared.
-    // Every group stores its fragments (GPS8 groups per ring slot); then group g < 4 FM adds
-    // row quad g % 4 of row fragment g / 4 (both column groups) over all eight groups and
-    // runs the epilogue for those rows -- up to eight waves instead of one reading and storing.
-    constexpr int GR = FM * FN * 4096;  // bytes of one group's fragments
-    constexpr int GPS8 = QB / GR;       // groups per ring slot
-    if constexpr (KW == 8 && NW == 1 && FN == 2 && (FM == 1 || FM == 2) && GPS8 >= 2 &&
-                  (8 + GPS8 - 1) / GPS8 <= (D < 4 ? D : 4)) {
-      const bool whole = row0 + BM <= act.rows && (cgb + BG) * 32 <= N && !accz && !rawacc && ntail == 0 &&
-                         (EPI != kEpiSwigluPair ||
-                          static_cast<size_t>(row0 + BM) * Nout <= static_cast<size_t>(swn & ~7));
-      if (whole) {
-        auto grp = [&](int g) -> v4i* {  // [fragment][quad][lane] as int4, GR bytes per group
-          const int sl = g / GPS8;
-          return reinterpret_cast<v4i*>((sl == 0 ? q0 : (sl == 1 ? q1 : (sl == 2 ? q2 : q3))) + (g % GPS8) * GR);
-        };
-        __syncthreads();
-        {
-          v4i* my = grp(kg);
-#pragma unroll
-          for (int f = 0; f < FM * FN; ++f)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const v16i& v = acc[P - 1][f / FN][f % FN];
-              my[(f * 4 + q) * 64 + lane] = v4i{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
-            }
-        }
-        __syncthreads();
-        if (kg >= FM * 4) return;  // 32-row tiles: four row quads, four waves
-        const int ai = kg >> 2, q = kg & 3;
-        v4i tot[FN];
-#pragma unroll
-        for (int bj = 0; bj < FN; ++bj) tot[bj] = v4i{0, 0, 0, 0};
-#pragma unroll
-        for (int g = 0; g < 8; ++g) {
-          const v4i* src = grp(g);
-#pragma unroll
-          for (int bj = 0; bj < FN; ++bj) {
-            const v4i t = src[((ai * FN + bj) * 4 + q) * 64 + lane];
-            tot[bj] = tot[bj] + t;
-          }
-        }
-        // rows rbase + e of this quad (fragment row 8 q + 4 (lane / 32) + e), columns col[bj]
-        const int rb = row0 + ai * 32 + 4 * (lane >> 5) + 8 * q;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int r = rb + e;
-          const size_t grow = static_cast<size_t>(r);
-          float val[FN];
-#pragma unroll
-          for (int bj = 0; bj < FN; ++bj) {
-            const int32_t sacc = tot[bj][e] + csum[bj];
-            if constexpr (MODE == kFixed) {
-              val[bj] = static_cast<float>(sacc) * invf;
-            } else {
-              const float den = srow[r - row0];
-              val[bj] = rcp_ok ? div_by_recip(static_cast<float>(sacc), den, srcp[r - row0])
-                               : static_cast<float>(sacc) / den;
-            }
-          }
-          if constexpr (EPI == kEpiSwigluPair) {
-            outz[grow * Nout + col[0]] = swiglu_of(val[0], val[1], false);
-          } else {
-#pragma unroll
-            for (int bj = 0; bj < FN; ++bj) {
-              const size_t o = grow * N + col[bj];
-              outz[o] = (EPI == kEpiAdd) ? addp[o] + val[bj] : val[bj];
-            }
-          }
-        }
-        return;
       }
-    }
-    // Two K-groups of two row fragments each (the long-prefill 128 x 128 tiles): the groups
-    // split the sum and the epilogue by row fragment. Group g keeps fragment g, sends its
-    // fragment 1 - g to the same wave of the other group through LDS and adds the one it
-    // receives (exact int32 sums: any order), then stores its own 32-row half of the tile.
-    if constexpr (KW2S) {
-      // (kept and sent fragments as compile-time indices: a run-time index into the
-      // accumulator array would put it in scratch memory)
-      auto exch = [&](auto keepc) {
-        constexpr int KEEP = decltype(keepc)::value, SEND = 1 - KEEP;
-        __syncthreads();
-        {
-          v4i* out = reinterpret_cast<v4i*>((KEEP == 0 ? (wave < 2 ? q0 : q1) : (wave < 2 ? q2 : q3)) +
-                                            (wave & 1) * (FN * 4 * 64 * 16));
-#pragma unroll
-          for (int bj = 0; bj < FN; ++bj)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const v16i& v = acc[P - 1][SEND][bj];
-              out[(bj * 4 + q) * 64 + lane] = v4i{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
-            }
-        }
-        __syncthreads();
-        {
-          const v4i* in = reinterpret_cast<const v4i*>((KEEP == 1 ? (wave < 2 ? q0 : q1) : (wave < 2 ? q2 : q3)) +
-                                                       (wave & 1) * (FN * 4 * 64 * 16));
-#pragma unroll
-          for (int bj = 0; bj < FN; ++bj)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const v4i t = in[(bj * 4 + q) * 64 + lane];
-#pragma unroll
-              for (int e = 0; e < 4; ++e) acc[P - 1][KEEP][bj][4 * q + e] += t[e];
-            }
-        }
-        if constexpr (KEEP == 1) {  // the kept fragment to slot 0: the epilogue runs on slot 0
-#pragma unroll
-          for (int bj = 0; bj < FN; ++bj) acc[P - 1][0][bj] = acc[P - 1][1][bj];
-        }
-      };
-      if (kg == 0) exch(std::integral_constant<int, 0>{});
-      else exch(std::integral_constant<int, 1>{});
-    } else {
-    // fragments per round: the most (up to all of them) for which every wave's fragments of
-    // groups 1..KW-1 fit the first min(D, 4) ring slots, GPS groups sharing a slot
-    constexpr int NS = D < 4 ? D : 4;
-    constexpr int FB = [] {
-      for (int fb = FM * FN; fb >= 1; --fb) {
-        const int gps = QB / (NW * fb * 4096);
-        if (gps >= 1 && (KW - 1 + gps - 1) / gps <= NS) return fb;
-      }
-      return 0;
-    }();
-    static_assert(FB >= 1, "the reduced groups fit the ring slots");
-    constexpr int GB = NW * FB * 4096;  // bytes of one group's round
-    constexpr int GPS = QB / GB;
-    auto red_slot = [&](int r) -> v4i* {  // [wave][fragment of the round][quad][lane] as int4
-      const int sl = (r - 1) / GPS, off = ((r - 1) % GPS) * GB;
-      return reinterpret_cast<v4i*>((sl == 0 ? q0 : (sl == 1 ? q1 : (sl == 2 ? q2 : q3))) + off);
-    };
-#pragma unroll
-    for (int f0 = 0; f0 < FM * FN; f0 += FB) {
       __syncthreads();
-      if (kg != 0) {
-        v4i* red = red_slot(kg);
+      {
+        const v4i* in = reinterpret_cast<const v4i*>(ring) + (SEND * 4 + wave) * XW;
 #pragma unroll
-        for (int f = f0; f < f0 + FB && f < FM * FN; ++f)
+        for (int bj = 0; bj < FN; ++bj)
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            const v16i& v = acc[P - 1][f / FN][f % FN];
-            red[((wave * FB + f - f0) * 4 + q) * 64 + lane] = v4i{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+            const v4i t = in[(bj * 4 + q) * 64 + lane];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[P - 1][KEEP][bj][4 * q + e] += t[e];
           }
       }
-      __syncthreads();
-      if (kg == 0) {
+      if constexpr (KEEP == 1) {  // the kept fragment to slot 0: the epilogue runs on slot 0
 #pragma unroll
-        for (int r = 1; r < KW; ++r) {
-          const v4i* red = red_slot(r);
-#pragma unroll
-          for (int f = f0; f < f0 + FB && f < FM * FN; ++f)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const v4i t = red[((wave * FB + f - f0) * 4 + q) * 64 + lane];
-#pragma unroll
-              for (int e = 0; e < 4; ++e) acc[P - 1][f / FN][f % FN][4 * q + e] += t[e];
-            }
-        }
+        for (int bj = 0; bj < FN; ++bj) acc[P - 1][0][bj] = acc[P - 1][1][bj];
       }
-    }
-    if (kg != 0) return;
-    }
+    };
+    if (kg == 0) exch(std::integral_constant<int, 0>{});
+    else exch(std::integral_constant<int, 1>{});
   }
 
   // with the two-group split each group stores one row fragment, held in slot 0, whose rows
   // are shifted by its group index
   constexpr int FME = KW2S ? 1 : FM;
   const int ash = KW2S ? kg : 0;
-  if (ksp > 1) {
-    // split-K: exact partial sums of this stage range, logical column order
-    int32_t* wp = wsp + (static_cast<size_t>(ks) * a.nmat + z) * act.rows * static_cast<size_t>(N);
-    const int Nh = N / 2;
-#pragma unroll
-    for (int bj = 0; bj < FN; ++bj) {
-      const int cg = cgb + wn * FN + bj;
-      const int o = (EPI == kEpiSwigluPair) ? ((cg & 1) ? Nh : 0) + (cg >> 1) * 32 + ol : cg * 32 + ol;
-      if (cg >= ng32 || o >= N) continue;
-#pragma unroll
-      for (int ai = 0; ai < FME; ++ai)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int row = row0 + (wm * FM + ai + ash) * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-          if (row >= act.rows) continue;
-          wp[static_cast<size_t>(row) * N + o] =
-              (MODE == kFixed) ? acc[0][ai][bj][i] * 256 + acc[P - 1][ai][bj][i] : acc[0][ai][bj][i];
-        }
-    }
-    return;
-  }
-
-  // epilogue: exact integer totals, dequantisation, output stage. The residual rows of
-  // all fragments are loaded in one batch before any store. Stored columns of this lane:
-  // one per group (NB = FN), or one per swiglu pair (its gate column; NB = FN / 2).
-  constexpr int NB = (EPI == kEpiSwigluPair) ? FN / 2 : FN;
-  constexpr int GS = (EPI == kEpiSwigluPair) ? 2 : 1;  // groups per stored column
-  bool cok[NB];
-#pragma unroll
-  for (int b = 0; b < NB; ++b) cok[b] = col[GS * b] < Nout;
-  float addv[FM][16][NB];
-  if (EPI == kEpiAdd) {
-#pragma unroll
-    for (int ai = 0; ai < FME; ++ai)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        int row = row0 + (wm * FM + ai + ash) * 32 + 4 * (lane >> 5) + 8 * (i >> 2) + (i & 3);
-        row = row < act.rows ? row : act.rows - 1;
-#pragma unroll
-        for (int b = 0; b < NB; ++b) addv[ai][i][b] = cok[b] ? addp[static_cast<size_t>(row) * N + col[b]] : 0.0f;
-      }
-  }
-  // Whole tile in range, no tail weights, no integer accumulator output, below the swiglu
-  // tail rule: one straight store per output with no per-element tests (the general path
-  // below measured several times slower per tile).
-  const bool fast = row0 + BM <= act.rows && (cgb + BG) * 32 <= N && !accz && !rawacc && ntail == 0 &&
+  // Whole tile in range, no tail weights, no integer accumulator output, no split, below the
+  // swiglu tail rule: one straight store per output with no per-element tests. The residual rows
+  // of all fragments are loaded in one batch before any store. Stored columns of this lane: one
+  // per group (NB = FN), or one per swiglu pair (its gate column; NB = FN / 2).
+  constexpr int NB = PAIR ? FN / 2 : FN;
+  const bool fast = ksp == 1 && row0 + BM <= act.rows && (cgb + BG) * 32 <= N && !accz && !rawacc && ntail == 0 &&
                     (EPI != kEpiSwigluPair || static_cast<size_t>(row0 + BM) * Nout <= static_cast<size_t>(swn & ~7));
   auto fast_epi = [&](auto use_rcp) {
 #pragma unroll
     for (int ai = 0; ai < FME; ++ai) {
       const int rbase = row0 + (wm * FM + ai + ash) * 32 + 4 * (lane >> 5);
+      float addv[16][NB];  // the fragment's residuals, all loaded before any is used
+      if constexpr (EPI == kEpiAdd) {
+        const float* ap = addp + static_cast<size_t>(rbase) * N + col[0];
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+#pragma unroll
+          for (int b = 0; b < NB; ++b) addv[i][b] = ap[static_cast<size_t>(8 * (i >> 2) + (i & 3)) * N + 32 * b];
+      }
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int r = rbase + 8 * (i >> 2) + (i & 3);
@@ -689,7 +669,7 @@ __global__ __launch_bounds__(64 * WM * WN * KW, (mfma_min_waves<MODE, EPI, WM, W
           if (EPI == kEpiSwigluPair)
             outz[grow * Nout + col[2 * b]] = swiglu_of(val[2 * b], val[2 * b + 1], false);
           else
-            outz[grow * N + col[b]] = (EPI == kEpiAdd) ? addv[ai][i][b] + val[b] : val[b];
+            outz[grow * N + col[b]] = (EPI == kEpiAdd) ? addv[i][b] + val[b] : val[b];
         }
       }
     }
@@ -699,49 +679,130 @@ __global__ __launch_bounds__(64 * WM * WN * KW, (mfma_min_waves<MODE, EPI, WM, W
     else fast_epi(std::false_type{});
     return;
   }
+  // Partial tiles, tails, accumulators, split-K partials: through LDS. Each wave turns its
+  // accumulators, one 32-row fragment at a time, into rows of 64 sums in its own part of the
+  // (free) ring, then takes them back as four neighbouring columns per lane: 16-byte accesses at
+  // any 4-byte alignment, one test per row, and a loop over the rows. Straight-line code for
+  // every accumulator with its tests and tails was bound by the instruction fetch: 64 x 300 x
+  // 6000 33 us per launch, now 14. (Whole tiles measured 3-5% slower this way: they keep the
+  // straight stores above.)
+  constexpr int ES = 72;  // row stride in words: the half waves' rows (four apart) on other banks
+  static_assert(FN == 2 && NW * KW * 32 * ES * 4 <= RB, "the waves' rows fit the ring");
+  int32_t* const T = reinterpret_cast<int32_t*>(ring) + wid * 32 * ES;
+  constexpr int LR = PAIR ? 8 : 16;   // lanes per row
+  constexpr int RI = 64 / LR;         // rows per iteration
+  constexpr int NC = PAIR ? 8 : 4;    // columns of this lane: four neighbours (and their up partners)
+  const int lc = 4 * (lane & (LR - 1));
+  const int ecol = (PAIR ? ((cgb + wn * FN) >> 1) : cgb + wn * FN) * 32 + lc;
+  const int nv = Nout - ecol;  // columns of this lane in range (>= 4: all)
+  int32_t cs[NC];
+  uint32_t tw[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int cc = ecol + (c & 3) + ((c & 4) ? Nout : 0);
+    cs[c] = (MODE == kFixed && ksp == 1) ? 128 * rsum[cc < N ? cc : N - 1] : 0;
+    tw[c] = tail_of(cc);
+  }
+  int32_t* const wp = wsp + (static_cast<size_t>(ks) * a.nmat + z) * arows * static_cast<size_t>(N);  // ksp > 1
+  auto put = [&](auto* base, size_t o, const auto* v) {
+    typedef std::remove_reference_t<decltype(*base)> E;
+    typedef E E4 __attribute__((ext_vector_type(4), aligned(4)));
+    if (nv >= 4) {
+      *reinterpret_cast<E4*>(base + o) = E4{v[0], v[1], v[2], v[3]};
+    } else {
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        if (k < nv) base[o + k] = v[k];
+    }
+  };
+  __syncthreads();
 #pragma unroll
   for (int ai = 0; ai < FME; ++ai) {
-    const int rbase = row0 + (wm * FM + ai + ash) * 32 + 4 * (lane >> 5);
-    float den[16];
-    if (MODE == kInt8) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) den[i] = srow[rbase - row0 + 8 * (i >> 2) + (i & 3)];
-    }
+    for (int bj = 0; bj < FN; ++bj)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int row = rbase + 8 * (i >> 2) + (i & 3);
-      if (row >= act.rows) continue;
+      for (int i = 0; i < 16; ++i)
+        T[(8 * (i >> 2) + 4 * (lane >> 5) + (i & 3)) * ES + 32 * bj + ol] =
+            (MODE == kFixed) ? acc[0][ai][bj][i] * 256 + acc[P - 1][ai][bj][i] : acc[0][ai][bj][i];
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const int fr0 = (wm * FM + ai + ash) * 32;  // the fragment's first row in the block
+#pragma unroll(PAIR ? 1 : 2)
+    for (int it = 0; it < 32 / RI; ++it) {
+      const int rl = it * RI + lane / LR, rb = fr0 + rl, row = row0 + rb;
+      if (row >= arows || nv <= 0) continue;
       const size_t grow = static_cast<size_t>(row);
-      const int32_t* ct = act.ct + (static_cast<size_t>(am) * act.rows + row) * 8;
-      int32_t tot[FN];
-      float val[FN];
+      int32_t s[NC];
 #pragma unroll
-      for (int bj = 0; bj < FN; ++bj) {
-        int32_t s = (MODE == kFixed) ? acc[0][ai][bj][i] * 256 + acc[P - 1][ai][bj][i] + csum[bj] : acc[0][ai][bj][i];
-        if (ntail && col[bj] < N)
-          for (int t = 0; t < ntail; ++t) s += static_cast<int32_t>(tailp[col[bj] * 8 + t]) * ct[t];
-        tot[bj] = s;
-        val[bj] = (MODE == kFixed) ? static_cast<float>(s) * invf : static_cast<float>(s) / den[i];
+      for (int h = 0; h < NC / 4; ++h) {
+        const v4i t = *reinterpret_cast<const v4i*>(T + rl * ES + 32 * h + lc);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) s[4 * h + k] = t[k];
       }
+      if (ksp > 1) {  // split-K: the exact partial sums of this stage range
+        put(wp, grow * N + ecol, s);
+        if (PAIR) put(wp, grow * N + Nout + ecol, s + NC - 4);
+        continue;
+      }
+      float res[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+      if constexpr (EPI == kEpiAdd) {
+        const float* ap = addp + grow * N + ecol;
+        if (nv >= 4) {
+          typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+          const f4u t = *reinterpret_cast<const f4u*>(ap);
 #pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        if (!cok[b]) continue;
-        if (EPI == kEpiSwigluPair) {
-          if (accz) {
-            accz[grow * N + col[2 * b]] = tot[2 * b];
-            accz[grow * N + col[2 * b + 1]] = tot[2 * b + 1];
-          }
-          if (rawacc) continue;
-          const size_t e = grow * Nout + col[2 * b];
-          outz[e] = swiglu_of(val[2 * b], val[2 * b + 1], static_cast<int64_t>(e) >= (swn & ~7));
+          for (int k = 0; k < 4; ++k) res[k] = t[k];
         } else {
-          const size_t e = grow * N + col[b];
-          if (accz) accz[e] = tot[b];
-          if (rawacc) continue;
-          outz[e] = (EPI == kEpiAdd) ? addv[ai][i][b] + val[b] : val[b];
+#pragma unroll
+          for (int k = 0; k < 3; ++k) res[k] = k < nv ? ap[k] : 0.0f;
         }
       }
+#pragma unroll
+      for (int c = 0; c < NC; ++c) s[c] += cs[c];
+      if (ntail) {
+        const int4 c0 = stct[2 * rb], c1 = stct[2 * rb + 1];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) s[c] += tail_term(c0, c1, tw[c]);
+      }
+      if (accz) {
+        put(accz, grow * N + ecol, s);
+        if (PAIR) put(accz, grow * N + Nout + ecol, s + NC - 4);
+      }
+      if (rawacc) continue;
+      float v[NC];
+      if constexpr (MODE == kFixed) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) v[c] = static_cast<float>(s[c]) * invf;
+      } else {
+        const float den = srow[rb];
+        if (rcp_ok) {
+          const float rcp = srcp[rb];
+#pragma unroll
+          for (int c = 0; c < NC; ++c) v[c] = div_by_recip(static_cast<float>(s[c]), den, rcp);
+        } else {
+#pragma unroll
+          for (int c = 0; c < NC; ++c) v[c] = static_cast<float>(s[c]) / den;
+        }
+      }
+      if constexpr (PAIR) {
+        const size_t o = grow * Nout + ecol;
+        const bool body = static_cast<int64_t>(o) + 3 < (swn & ~7);
+        float r[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          r[k] = body ? swiglu_of(v[k], v[4 + k], false)
+                      : swiglu_of(v[k], v[4 + k], static_cast<int64_t>(o) + k >= (swn & ~7));
+        put(outz, o, r);
+      } else {
+        if constexpr (EPI == kEpiAdd) {
+#pragma unroll
+          for (int k = 0; k < 4; ++k) v[k] = res[k] + v[k];
+        }
+        put(outz, grow * N + ecol, v);
+      }
     }
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   }
 }
 
@@ -839,36 +900,44 @@ constexpr int kStageKQ = 2;
 template <int MODE, int EPI, int TM, int TN, int KQ, int KW, int FM = 2>
 bool mfma_launch(const GemmArgs& a, const ActBuf& act, dim3 grid, hipStream_t s) {
   constexpr int WM = TM, WN = TN, FN = 2;
-  constexpr int bytes =
-      ring_depth<MODE, WM, WN, FM, FN, KQ, KW>() * KW * stage_bytes<MODE, WM, WN, FM, FN, KQ>() + row_scale_bytes<MODE, WM, FM>();
+  constexpr int ring = ring_depth<MODE, WM, WN, FM, FN, KQ, KW>() * KW * stage_bytes<MODE, WM, WN, FM, FN, KQ>();
+  constexpr int sums = KW == 8 ? 8 * FM * FN * 4096 : 0;
+  constexpr int bytes = (ring > sums ? ring : sums) + row_scale_bytes<MODE, WM, FM>();
   if (bytes > lds_limit()) return false;
   k_mfma<MODE, EPI, WM, WN, FM, FN, KQ, KW><<<grid, dim3(64 * WM * WN * KW), 0, s>>>(a, act);
   return true;
 }
 
-// Tile shape: 64 rows for short row ranges (batched decode), else 128; 256 columns when
-// that still gives every CU a block (all blocks of all matrices), else 128. Then K is
-// split in powers of two until there are 128 blocks (each split >= 4 stages). A split GEMM
-// of 49-64 rows with K <= 6912 and enough tiles (at least kKGroupTiles 64 x 128 tiles, or
-// at least 64 32 x 64 tiles, or at most 64 stages) runs instead on tiles of eight K-groups
-// in one block (kw), whose partial tiles meet in LDS: no partials through memory and no
-// split-K epilogue launch; 8-32 rows take 32 x 64 such tiles (K <= 4096, or K <= 6912
-// with at least 32 tiles).
+// Tile shape. Launches of up to a few hundred tiles: eight K-groups of one wave in a block
+// (kw = 8), whose partial tiles meet in LDS: every SIMD has two waves on an eighth of the stages
+// each. 32 x 64 tiles (fm = 1) while they fit one block per CU, then 64 x 64 tiles while those
+// do, then 64 x 64 (FixedQ510) or 32 x 64 (Int8Absmax, whose blocks share a CU) while they take
+// two to three rounds. Against the 128-row tiles or splits over K with a second kernel that
+// such launches took before (us per BitLinear call): 100 x 1031 x 1333 FixedQ510 16.0 -> 9.6,
+// 128 x 513 x 5000 18.1 -> 9.7, 256 x 2048 x 6000 30.2 -> 19.2, 1024 x 4098 x 2000 43.4 ->
+// 38.1, Int8Absmax 256 x 1024 x 5632 23.3 -> 12.9, 512 x 6912 x 2560 40.1 -> 31.3; past the
+// limits 512 x 513 x 5000 FixedQ510 17.1 -> 20.9 (64 x 64), 384 x 1024 x 5632 Int8Absmax 14.4 ->
+// 17.4 (32 x 64). Below K = 512 the second round does not pay (384 x 64 x 3000: 10.9 -> 11.9).
+// Above that: 128-row tiles (64 rows for the few-row launches of very wide matrices), 256
+// columns when that still gives every CU a block (all blocks of all matrices), else 128. For K
+// beyond 6912 (stages beyond kGroupStages), K is split in powers of two until there are 128
+// blocks (each split >= 4 stages): the eight waves of one block would walk too many stages.
 struct Plan {
   int wm, wn, ksplit, kw;
   int fm = 2;  // 32-row fragments per wave (1: 32-row tiles)
 };
-static bool kw8_rows32() {
-  static const bool on = [] {
-    const char* e = std::getenv("MMF_KW8_32");
-    return !(e && e[0] == '0');
-  }();
-  return on;
-}
-constexpr int kKGroupTiles = 48;
+constexpr int kGroupStages = 216;
 
 Plan plan_of(const GemmArgs& a) {
   const int nz = (a.epi == kEpiSwigluPair) ? 1 : a.nmat;
+  const int nst = a.p[0].g.Lc / 8;
+  const int t32 = tiles_of<1, 1, 1>(a) * nz, t64 = tiles_of<1, 1>(a) * nz;
+  if (nst <= kGroupStages) {
+    const bool two = a.p[0].g.K >= 512;  // a second round of tiles
+    if (t32 <= 256) return Plan{1, 1, 1, 8, 1};
+    if (t64 <= 256 || (two && a.mode == kFixed && t64 <= 512)) return Plan{1, 1, 1, 8, 2};
+    if (two && a.mode == kInt8 && t32 <= 768) return Plan{1, 1, 1, 8, 1};
+  }
   Plan p{a.rows <= 64 ? 1 : 2, 4, 1, 1};
   if (p.wm == 1 ? tiles_of<1, 4>(a) * nz < 256 : tiles_of<2, 4>(a) * nz < 256) p.wn = 2;
   // FixedQ510 (two int8 passes per tile) over 128-row tiles: 128 x 128 tiles throughout.
@@ -888,36 +957,8 @@ Plan plan_of(const GemmArgs& a) {
                                : (p.wn == 4 ? tiles_of<2, 4>(a) : tiles_of<2, 2>(a))) * nz;
   // split K until there are 128 blocks (one per two CUs; more splits measured slower, the
   // partial traffic growing with the split count), keeping >= 4 stages per split
-  const int nst = a.p[0].g.Lc / 8;
-  while (tiles * p.ksplit < 128 && nst / (2 * p.ksplit) >= 4 && p.ksplit < 16) p.ksplit *= 2;
-  const int t32 = tiles_of<1, 1, 1>(a) * nz;  // 32 x 64 tiles
-  // 8-32 rows: 32 x 64 tiles of eight K-groups where K <= 4096 (16-row op calls: 2048 x
-  // 11264 15.8 -> 11.6 us, 1024 x 1024 10.5 -> 9.6 us per call), or over 16 rows K <= 6912
-  // with at least 32 tiles (the 1.3B down projection, K = 5632: 12.2 us per launch against
-  // 9.4 us for the split plus 2.0 us for its epilogue launch, whose writes also delayed the
-  // next launch by 2.4 us; at 16 rows the split stays faster, 15.5 against 17.2 us)
-  if (kw8_rows32() && a.rows >= 8 && a.rows <= 32 && p.ksplit > 1 && nst >= 16 &&
-      (nst <= 64 || (nst <= 216 && t32 >= 32 && a.rows > 16))) {
-    p = Plan{1, 1, 1, 8, 1};
-    return p;
-  }
-  if (p.wm == 1 && a.rows > 48 && p.ksplit > 1 && nst >= 16 && nst <= 216 &&
-      (tiles >= kKGroupTiles || nst <= 64 || t32 >= 64)) {
-    // (a 4-wave-wide tile never splits: it has >= 256 tiles) tiles of eight K-groups, one
-    // wave each, 32-position stages: twice the blocks of 64 x 128 tiles with four K-groups
-    // of two waves, each wave a quarter of the chain of stages (64 rows, FixedQ510: i/f/g
-    // 2560 x 3 x 2560 18.1 -> 16.3 us, gate/up 2560 x 13824 20.1 -> 18.6 us per launch in a
-    // step, before the shared epilogue below). 32 x 64 tiles where they still fit one block
-    // per CU: twice the blocks, half the activation rows streamed through each CU (2.7B x 64
-    // FixedQ510 step, per launch: i/f/g 11.0 -> 8.2 us, o 12.9 -> 9.8 us; the down
-    // projection, K = 6912, 14.5 us against 10.7 us for the split plus 5.1 us for its
-    // epilogue launch, whose writes also delayed the next launch by 3.5 us); else 64 x 64
-    // (gate/up: 432 32 x 64 tiles would take two rounds, 18.0 against 11.8 us).
-    p.kw = 8;
-    p.wn = 1;
-    p.ksplit = 1;
-    if (t32 <= 256) p.fm = 1;
-  }
+  if (nst > kGroupStages)
+    while (tiles * p.ksplit < 128 && nst / (2 * p.ksplit) >= 4 && p.ksplit < 16) p.ksplit *= 2;
   // 128 x 128 tiles at one block per CU (the 2048-column o/down GEMMs of a long prefill):
   // two K-groups per block give each SIMD two waves instead of one, with the same tile
   // and operand traffic
@@ -990,7 +1031,7 @@ hipError_t launch_pack_mfma(const uint32_t* pk, const Geom& g, bool pair, uint32
 }
 
 size_t gemm_workspace_bytes(const GemmArgs& a) {
-  if (a.mode == kFloat || mfma_min_rows() <= 0 || a.rows < mfma_min_rows()) return 0;
+  if (a.mode == kFloat || !int_mfma_rows(a.mode, a.rows, a.p[0].g.K)) return 0;
   const Plan p = plan_of(a);
   if (p.ksplit == 1) return 0;
   return static_cast<size_t>(p.ksplit) * a.nmat * a.rows * static_cast<size_t>(a.p[0].g.N) * sizeof(int32_t);

@@ -2212,16 +2212,17 @@ int float_mfma_min_rows() {
   return v;
 }
 
-int mfma_min_rows() {
-  static const int v = [] {
+bool int_mfma_rows(Mode mode, int rows, int K) {
+  static const int min_rows = [] {
     const char* e = std::getenv("MMF_MFMA_MIN_ROWS");
-    return e ? std::atoi(e) : 8;
+    return e ? std::atoi(e) : -1;
   }();
-  return v;
+  if (min_rows >= 0) return min_rows > 0 && rows >= min_rows;
+  return rows >= (mode == kFixed ? 3 : 4) || static_cast<int64_t>(rows) * K >= 1024;
 }
 
 hipError_t launch_gemm(const GemmArgs& a, const ActBuf& act, hipStream_t s) {
-  if (a.mode != kFloat && mfma_min_rows() > 0 && a.rows >= mfma_min_rows()) {
+  if (a.mode != kFloat && int_mfma_rows(a.mode, a.rows, a.p[0].g.K)) {
     // (the matrix-core kernel addresses a matrix's planes and weights with 31-bit offsets)
     bool ok = 2 * act.qplane() <= 0x7FFFFFFFu;
     for (int z = 0; z < (a.epi == kEpiSwigluPair ? 1 : a.nmat); ++z)
