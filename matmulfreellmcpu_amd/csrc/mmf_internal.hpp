@@ -265,7 +265,7 @@ int float_mfma_min_rows();
 // stream_state = true: rows are independent streams, state [rows, H].
 // keep_gates: f is overwritten with the gated forget values and scan_out receives the
 // recurrence input ([rows, H]; required for a time scan of more than one row). Without it,
-// a time scan with H % 16 == 0 computes the gates inside the scan kernel and leaves f and
+// a time scan computes the gates inside the scan kernel and leaves f and
 // scan_out untouched.
 hipError_t launch_mixer(const float* i, float* f, float* scan_out, float* recur, float* state,
                         const float* lb, int rows, int H, bool stream_state, bool keep_gates, hipStream_t s);

@@ -1533,49 +1533,10 @@ __global__ void k_gate(const float* __restrict__ i, float* __restrict__ f, float
   }
 }
 
-// The recurrence state = fma(g, state, in) (simd.hpp:335-357) down each column, in time
-// order. One thread per column; the g and in values of the next kScanU steps are loaded
-// while the current kScanU steps are computed.
-constexpr int kScanU = 64;
-
-__global__ __launch_bounds__(64) void k_scan_seq(const float* __restrict__ g, const float* __restrict__ in,
-                                                 float* __restrict__ recur, float* __restrict__ state, int rows,
-                                                 int H) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= H) return;
-  float s = state[c];
-  float gc[kScanU], ic[kScanU], gn[kScanU], inx[kScanU];
-  auto load = [&](int t0, float* gd, float* id) {
-#pragma unroll
-    for (int u = 0; u < kScanU; ++u) {
-      const int t = t0 + u < rows ? t0 + u : rows - 1;
-      gd[u] = g[static_cast<size_t>(t) * H + c];
-      id[u] = in[static_cast<size_t>(t) * H + c];
-    }
-  };
-  load(0, gc, ic);
-  for (int t0 = 0; t0 < rows; t0 += kScanU) {
-    if (t0 + kScanU < rows) load(t0 + kScanU, gn, inx);
-#pragma unroll
-    for (int u = 0; u < kScanU; ++u) {
-      if (t0 + u < rows) {
-        s = __builtin_fmaf(gc[u], s, ic[u]);
-        recur[static_cast<size_t>(t0 + u) * H + c] = s;
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < kScanU; ++u) {
-      gc[u] = gn[u];
-      ic[u] = inx[u];
-    }
-  }
-  state[c] = s;
-}
-
 // The recurrence of several independent sequences stacked as row segments (the prompts of
 // the serving streams): segment b = rows [off[b], off[b + 1]) starts from state b
 // (state + b * H) and leaves its last value there. One thread per (column, segment); each
-// segment is scanned in time order exactly as k_scan_seq scans one sequence.
+// segment is scanned in time order exactly as k_scan_ring scans one sequence.
 // GATE: g and in are the raw f and i projections and the gate math (k_gate's arithmetic,
 // no element tail since H % 8 == 0) runs on each step beside the chain.
 template <bool GATE>
@@ -1622,7 +1583,8 @@ __global__ void k_gather_rows(const float* __restrict__ x, const int* __restrict
   for (int k = threadIdx.x; k < K; k += blockDim.x) dst[k] = src[k];
 }
 
-// The recurrence for H % C == 0 (C = 4, 8 or 16 columns per block), staged through LDS so
+// The recurrence state = fma(g, state, in) (simd.hpp:335-357) down each column, in time order
+// (C = 4, 8 or 16 columns per block), staged through LDS so
 // that enough bytes are in flight: a block owns C columns and walks time in tiles of kScTT
 // steps. Waves by role: wave 0 runs the C column chains (state = fma(g, state, in), in
 // time order) at raised issue priority; waves 1-4 fill a ring of kScNR tiles of g and in by
@@ -1643,28 +1605,40 @@ constexpr int scan_ring_depth() {
 
 typedef __attribute__((address_space(3))) void lds_void_t;
 
-template <int C>
+// ANY (a width that is no multiple of C, or rows off 16-byte alignment): transfers of 4 bytes per
+// lane, 64 / C steps x C columns each, columns past the last repeating it (never stored).
+template <int C, bool ANY>
+constexpr int scan_transfers() {  // per array and tile
+  return ANY ? kScTT * C / 64 : kScTT * C / 256;
+}
+template <int C, bool ANY>
 __device__ __forceinline__ void scan_issue(const float* g, const float* in, float* ring, int tile, int slot,
                                            int T, int H, int c0, int lw, int lane) {
-  constexpr int TA = kScTT * C / 256;  // transfers per array per tile
+  constexpr int TA = scan_transfers<C, ANY>();
   constexpr int LPW = 2 * TA / 4;      // transfers per loader wave per tile
-  constexpr int SPT = 256 / C;         // steps per transfer
-  constexpr int LPR = C / 4;           // lanes per step row
+  constexpr int LPR = ANY ? C : C / 4; // lanes per step row
+  constexpr int SPT = 64 / LPR;        // steps per transfer
 #pragma unroll
   for (int i = 0; i < LPW; ++i) {
     const int idx = lw * LPW + i, arr = idx / TA, q = idx % TA;
     int t = tile * kScTT + SPT * q + lane / LPR;
     t = t < T ? t : T - 1;
-    const float* src = (arr ? in : g) + static_cast<size_t>(t) * H + c0 + 4 * (lane % LPR);
     float* dst = ring + ((slot * 2 + arr) * kScTT + SPT * q) * C;
-    __builtin_amdgcn_global_load_lds(src, (lds_void_t*)dst, 16, 0, 0);
+    if constexpr (ANY) {
+      const int c = c0 + lane % LPR;
+      const float* src = (arr ? in : g) + static_cast<size_t>(t) * H + (c < H ? c : H - 1);
+      __builtin_amdgcn_global_load_lds(src, (lds_void_t*)dst, 4, 0, 0);
+    } else {
+      const float* src = (arr ? in : g) + static_cast<size_t>(t) * H + c0 + 4 * (lane % LPR);
+      __builtin_amdgcn_global_load_lds(src, (lds_void_t*)dst, 16, 0, 0);
+    }
   }
 }
 
 // GATE: g and in are the raw f and i projections, and the conversion applies the gate math
 // (sigmoid, lower bound, swiglu; hgrn_model.cpp:113-124, the same functions as k_gate), so
-// the gated values never go through memory. Element tail rules do not arise: this kernel
-// requires H % 16 == 0.
+// the gated values never go through memory. The SIMD tail rule over all T x H elements arises
+// only in the ANY form (else H % 8 == 0).
 //
 // Each iteration k: the loaders issue the transfers of tile k + kScNR - 1; waves 1 .. 14
 // convert tile k + 1 from the ring (step-major, as loaded) into column-major rows GT / IT
@@ -1684,15 +1658,15 @@ __device__ __forceinline__ void scan_issue(const float* g, const float* in, floa
 // Tile k + 1 must then be in LDS at the barrier of iteration k, and an extra first iteration
 // converts tile 0. A partial last tile is chained one step at a time by the segment-0 lanes,
 // which store it themselves.
-template <bool GATE, int C, int kScNR = scan_ring_depth<C>()>
+template <bool GATE, int C, bool ANY, int kScNR = scan_ring_depth<C>()>
 __global__ __launch_bounds__(64 * kScWaves) void k_scan_ring(const float* __restrict__ g, const float* __restrict__ in,
                                                              const float* __restrict__ lb, float* __restrict__ recur,
                                                              float* __restrict__ state, int T, int H) {
   static_assert(C == 4 || C == 8 || C == 16, "4, 8 or 16 columns per block");
   constexpr int NCONV = kScWaves - 1 - kScStoreWaves;  // converting waves 1 .. NCONV
   static_assert((64 * NCONV) % C == 0, "a converting lane keeps its column");
-  static_assert((kScNR - 2) * kScTT * C / 512 < 64, "outstanding transfers per loader wave");
-  constexpr int LPW = kScTT * C / 512;  // transfers per loader wave per tile
+  constexpr int LPW = scan_transfers<C, ANY>() / 2;  // transfers per loader wave per tile
+  static_assert((kScNR - 2) * LPW < 64, "outstanding transfers per loader wave");
   constexpr int NSEG = 64 / C, SL = kScTT / NSEG;
   constexpr int LT = kScTT + 36;  // column row: the tile and a pad against bank conflicts
   extern __shared__ __align__(16) float sm[];
@@ -1702,7 +1676,7 @@ __global__ __launch_bounds__(64 * kScWaves) void k_scan_ring(const float* __rest
   float* ST = IT + 3 * C * LT;               // [2][64] starting states of the segments (tile & 1)
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   // column group: XCD-contiguous when the groups split evenly over the 8 XCDs
-  const int ngrp = H / C, b = blockIdx.x;
+  const int ngrp = ANY ? gridDim.x : H / C, b = blockIdx.x;
   const int grp = (ngrp % 8 == 0) ? (b & 7) * (ngrp / 8) + (b >> 3) : b;
   const int c0 = grp * C;
   const int ntiles = (T + kScTT - 1) / kScTT;
@@ -1713,15 +1687,17 @@ __global__ __launch_bounds__(64 * kScWaves) void k_scan_ring(const float* __rest
   const int sq0 = (wave - (kScWaves - kScStoreWaves)) * SQ;
   // chain and store waves: lane (cl, sg)
   const int cl = lane / NSEG, sg = lane % NSEG;
-  float s = (wave == 0 && sg == 0) ? state[c0 + cl] : 0.0f;
+  const bool live = !ANY || c0 + cl < H;  // this chain or store lane's column exists
+  float s = (wave == 0 && sg == 0 && state && live) ? state[c0 + cl] : 0.0f;
   // the chain is the block's critical path: its instructions issue ahead of the conversion
   // sharing its SIMD
   if (wave == 0) __builtin_amdgcn_s_setprio(3);
   // the column a converting lane handles is fixed (64 x NCONV lanes, C columns per step row)
   const int ccol = (threadIdx.x - 64) % C;
-  const float lbc = (GATE && conv && lb) ? lb[c0 + ccol] : 0.0f;
+  const float lbc = (GATE && conv && lb) ? lb[ANY && c0 + ccol >= H ? H - 1 : c0 + ccol] : 0.0f;
+  const size_t body = (static_cast<size_t>(T) * H) & ~static_cast<size_t>(7);  // ANY: the gate math's tail rule
   if (loader)
-    for (int t = 0; t < kScNR - 1 && t < ntiles; ++t) scan_issue<C>(g, in, ring, t, t, T, H, c0, wave - 1, lane);
+    for (int t = 0; t < kScNR - 1 && t < ntiles; ++t) scan_issue<C, ANY>(g, in, ring, t, t, T, H, c0, wave - 1, lane);
   for (int k = -1; k <= ntiles; ++k) {
     // this wave's LDS writes (converted tiles, starting states) have landed before the
     // barrier publishes them
@@ -1736,7 +1712,7 @@ __global__ __launch_bounds__(64 * kScWaves) void k_scan_ring(const float* __rest
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     if (loader && k >= 0 && k + kScNR - 1 < ntiles)
-      scan_issue<C>(g, in, ring, k + kScNR - 1, (k + kScNR - 1) % kScNR, T, H, c0, wave - 1, lane);
+      scan_issue<C, ANY>(g, in, ring, k + kScNR - 1, (k + kScNR - 1) % kScNR, T, H, c0, wave - 1, lane);
     if (conv && k + 1 < ntiles) {
       // tile k + 1 into column-major rows (GATE: g' = sigmoid(f), then the lower bound;
       // in' = swiglu(i, 1 - g'))
@@ -1747,12 +1723,13 @@ __global__ __launch_bounds__(64 * kScWaves) void k_scan_ring(const float* __rest
       const int n = min(kScTT, T - (k + 1) * kScTT);
       for (int e = threadIdx.x - 64; e < n * C; e += 64 * NCONV) {
         float gg = Gr[e], ii = Ir[e];
-        if (GATE) {
-          gg = sigmoid_of(gg, false);
-          if (lb) gg = __builtin_fmaf(1.0f - lbc, gg, lbc);
-          ii = swiglu_of(ii, 1.0f - gg, false);
-        }
         const int st = e / C;
+        if (GATE) {
+          const bool tail = ANY && (static_cast<size_t>(k + 1) * kScTT + st) * H + c0 + ccol >= body;
+          gg = sigmoid_of(gg, tail);
+          if (lb) gg = __builtin_fmaf(1.0f - lbc, gg, lbc);
+          ii = swiglu_of(ii, 1.0f - gg, tail);
+        }
         Gc[st] = gg;
         Ic[st] = ii;
       }
@@ -1793,7 +1770,7 @@ __global__ __launch_bounds__(64 * kScWaves) void k_scan_ring(const float* __rest
         float* out = recur + static_cast<size_t>(k) * kScTT * H + c0 + cl;
         for (int t = 0; t < n; ++t) {
           s = __builtin_fmaf(Gc[t], s, Ic[t]);
-          out[static_cast<size_t>(t) * H] = s;
+          if (live) out[static_cast<size_t>(t) * H] = s;
         }
       }
     }
@@ -1825,11 +1802,11 @@ __global__ __launch_bounds__(64 * kScWaves) void k_scan_ring(const float* __rest
         v[3] = r;
 #pragma unroll
         for (int c = 0; c < 4; ++c)
-          if (4 * u + c >= sq0 && 4 * u + c < sq0 + SQ) out[static_cast<size_t>(4 * u + c) * H] = v[c];
+          if (4 * u + c >= sq0 && 4 * u + c < sq0 + SQ && live) out[static_cast<size_t>(4 * u + c) * H] = v[c];
       }
     }
   }
-  if (wave == 0 && sg == 0) state[c0 + cl] = s;
+  if (wave == 0 && sg == 0 && state && live) state[c0 + cl] = s;
 }
 
 __global__ void k_embed(const float* __restrict__ emb, const int64_t* __restrict__ ids,
@@ -1877,6 +1854,84 @@ __global__ void k_rownorm(const float* __restrict__ x, const float* __restrict__
   }
 }
 
+// The same with eight consecutive elements per thread and group (t = tid + 256 g: chain position t
+// of every chain), every global input loaded once at entry as 16-byte accesses of any 4-byte
+// alignment, the row kept in registers between the norm chain and the output; t = nb is the tail
+// group. Arithmetic and order are k_rownorm's, which serves rows longer than 8 * 256 * MAXG.
+// Bound by a row's serial phases (load, chain of K / 8 steps, store); 2000 x 2048 10.5 -> 8.1 us
+// (swish gate 14.1 -> 10.6), 1000 x 2056 8.7 -> 6.6, against the element-by-element kernel.
+template <int MAXG, bool SW>
+__global__ __launch_bounds__(256) void k_rownorm8(const float* __restrict__ x, const float* __restrict__ o,
+                                                  const float* __restrict__ w, float* __restrict__ y, int cols,
+                                                  float eps) {
+  extern __shared__ __align__(16) float smem[];
+  const int K = cols, K8 = K & ~7, nb = K8 / 8, nt = K - K8, Lc = nb > 0 ? (nb + 15) / 16 * 16 : 16;
+  const int LS = lds_stride(Lc), L32 = (Lc + 31) / 32 * 32, tid = threadIdx.x;
+  float* X = smem;
+  float* red = X + 8 * LS + 8;
+  const size_t r0 = static_cast<size_t>(blockIdx.x) * K;
+  auto ld8 = [&](const float* p, int t, float* e) {
+    if (t < nb) {
+      const f4u l = reinterpret_cast<const f4u*>(p + 8 * t)[0], h = reinterpret_cast<const f4u*>(p + 8 * t)[1];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        e[c] = l[c];
+        e[4 + c] = h[c];
+      }
+    } else {
+#pragma unroll
+      for (int c = 0; c < 8; ++c) e[c] = p[K8 + (c < nt ? c : 0)];
+    }
+  };
+  const int G = nb + (nt > 0 ? 1 : 0);
+  float xv[MAXG][8], wv[MAXG][8], ov[SW ? MAXG : 1][8];
+#pragma unroll
+  for (int g = 0; g < MAXG; ++g) {
+    const int t = tid + 256 * g;
+    if (t >= G) continue;
+    ld8(x + r0, t, xv[g]);
+    ld8(w, t, wv[g]);
+    if constexpr (SW) ld8(o + r0, t, ov[g]);
+  }
+  for (int j = 0; j < 8; ++j)
+    for (int t = nb + tid; t < L32; t += 256) X[j * LS + t] = 0.0f;
+  for (int t = nt + tid; t < 8; t += 256) X[8 * LS + t] = 0.0f;
+#pragma unroll
+  for (int g = 0; g < MAXG; ++g) {
+    const int t = tid + 256 * g;
+    if (t >= G) continue;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      if (t < nb) X[c * LS + t] = xv[g][c];
+      else if (c < nt) X[8 * LS + c] = xv[g][c];
+    }
+  }
+  __syncthreads();
+  if (tid < 64) __builtin_amdgcn_s_setprio(3);
+  const float r = rstd_of(block_sumsq_ring(X, Lc, LS, nt, red), K, eps);
+  if (tid < 64) __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+  for (int g = 0; g < MAXG; ++g) {
+    const int t = tid + 256 * g;
+    if (t >= G) continue;
+    float v[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      v[c] = (xv[g][c] * r) * wv[g][c];
+      if (SW) v[c] = v[c] * silu_of(ov[SW ? g : 0][c], t >= nb);
+    }
+    float* yo = y + r0 + 8 * t;
+    if (t < nb) {
+      reinterpret_cast<f4u*>(yo)[0] = f4u{v[0], v[1], v[2], v[3]};
+      reinterpret_cast<f4u*>(yo)[1] = f4u{v[4], v[5], v[6], v[7]};
+    } else {
+#pragma unroll
+      for (int c = 0; c < 7; ++c)
+        if (c < nt) yo[c] = v[c];
+    }
+  }
+}
+
 __global__ void k_argmax_rows(const float* __restrict__ lg, int V, int64_t* __restrict__ ids) {
   __shared__ unsigned long long red[16];
   const float* r = lg + static_cast<size_t>(blockIdx.x) * V;
@@ -1917,25 +1972,18 @@ __global__ void k_quant_rows(const float* __restrict__ y, int32_t* __restrict__ 
   }
 }
 
-__global__ void k_swiglu(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ out,
-                         size_t n) {
+// Four elements per thread (16-byte accesses, at any 4-byte alignment); bound by memory.
+__global__ __launch_bounds__(256) void k_swiglu(const float* __restrict__ a, const float* __restrict__ b,
+                                                float* __restrict__ out, size_t n) {
   const size_t body = n & ~static_cast<size_t>(7);
-  for (size_t e = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; e < n;
-       e += static_cast<size_t>(gridDim.x) * blockDim.x)
-    out[e] = swiglu_of(a[e], b[e], e >= body);
-}
-
-__global__ void k_scan(const float* __restrict__ i, const float* __restrict__ f, float* __restrict__ out,
-                       float* __restrict__ state, int T, int D) {
-  const int d = blockIdx.x * blockDim.x + threadIdx.x;
-  if (d >= D) return;
-  float s = state ? state[d] : 0.0f;
-  for (int t = 0; t < T; ++t) {
-    const size_t e = static_cast<size_t>(t) * D + d;
-    s = __builtin_fmaf(f[e], s, i[e]);
-    out[e] = s;
+  const size_t e = 4 * (blockIdx.x * static_cast<size_t>(256) + threadIdx.x);
+  if (e < body) {  // (body is a multiple of 4)
+    const f4u x = *reinterpret_cast<const f4u*>(a + e), y = *reinterpret_cast<const f4u*>(b + e);
+    *reinterpret_cast<f4u*>(out + e) = f4u{swiglu_of(x[0], y[0], false), swiglu_of(x[1], y[1], false),
+                                           swiglu_of(x[2], y[2], false), swiglu_of(x[3], y[3], false)};
+  } else {
+    for (size_t k = e; k < n && k < e + 4; ++k) out[k] = swiglu_of(a[k], b[k], true);
   }
-  if (state) state[d] = s;
 }
 
 }  // namespace
@@ -2238,20 +2286,33 @@ hipError_t launch_gemm(const GemmArgs& a, const ActBuf& act, hipStream_t s) {
 }
 
 // Columns per k_scan_ring block: 8, so that H / 8 blocks (256 at H = 2048) cover the CUs;
-// the two blocks of a 64-byte line sit on one XCD and share its L2.
+// the two blocks of a 64-byte line sit on one XCD and share its L2. Widths that are no multiple
+// of 8, or addresses off 16 bytes, take the 4-byte transfers.
 template <bool GATE>
 static hipError_t scan_ring_launch(const float* g, const float* in, const float* lb, float* recur, float* state,
                                    int rows, int H, hipStream_t s) {
-  auto go = [&](auto cc) {
-    constexpr int C = decltype(cc)::value;
+  constexpr int C = 8;
+  const int groups = (H + C - 1) / C;
+  auto go = [&](auto any, auto nr) {
+    constexpr int NR = decltype(nr)::value;
     const size_t lds =
-        (static_cast<size_t>(scan_ring_depth<C>()) * 2 * kScTT * C + 6 * static_cast<size_t>(C) * (kScTT + 36) +
-         128) *
-        sizeof(float);
-    k_scan_ring<GATE, C><<<H / C, 64 * kScWaves, lds, s>>>(g, in, lb, recur, state, rows, H);
+        (static_cast<size_t>(NR) * 2 * kScTT * C + 6 * static_cast<size_t>(C) * (kScTT + 36) + 128) * sizeof(float);
+    k_scan_ring<GATE, C, decltype(any)::value, NR>
+        <<<groups, 64 * kScWaves, lds, s>>>(g, in, lb, recur, state, rows, H);
     return hipGetLastError();
   };
-  return go(std::integral_constant<int, 8>{});
+  // beyond one block per CU: a ring of 5 tiles (72 KB) lets two share a CU instead of running in
+  // two rounds (1000 x 2056: 25 -> 19 us); with the gate math in the block, which fills the CU's
+  // issue slots, that measured slower (4600 x 2560: 94 -> 98 us)
+  constexpr int NR = scan_ring_depth<C>();
+  auto depth = [&](auto any) {
+    if constexpr (!GATE) {
+      if (groups > 256) return go(any, std::integral_constant<int, 5>{});
+    }
+    return go(any, std::integral_constant<int, NR>{});
+  };
+  if (H % C == 0 && aligned16(g) && aligned16(in)) return depth(std::false_type{});
+  return depth(std::true_type{});
 }
 
 // Chunked parallel scan of the prefill recurrence (float mode, opt-in; not the reference's
@@ -2376,25 +2437,15 @@ hipError_t launch_scan_chunked(const float* i, const float* f, const float* lb, 
 
 hipError_t launch_mixer(const float* i, float* f, float* scan_out, float* recur, float* state,
                         const float* lb, int rows, int H, bool stream_state, bool keep_gates, hipStream_t s) {
-  if (!stream_state && !keep_gates && rows > 1 && H % 16 == 0 &&
-      ((reinterpret_cast<uintptr_t>(i) | reinterpret_cast<uintptr_t>(f) | reinterpret_cast<uintptr_t>(recur)) & 15) == 0) {
-    // one kernel: the gate math runs inside the scan on each tile (k_scan_ring<true, C>)
-    return scan_ring_launch<true>(f, i, lb, recur, state, rows, H, s);
-  }
+  // one kernel: the gate math runs inside the scan on each tile
+  if (!stream_state && !keep_gates && rows > 1) return scan_ring_launch<true>(f, i, lb, recur, state, rows, H, s);
   if (!stream_state && scan_out && rows > 1) {
     const size_t n = static_cast<size_t>(rows) * H;
     const int blocks = static_cast<int>(std::min<size_t>((n + 255) / 256, 16384));
     k_gate<<<blocks, 256, 0, s>>>(i, f, scan_out, lb, rows, H);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const bool aligned = ((reinterpret_cast<uintptr_t>(f) | reinterpret_cast<uintptr_t>(scan_out) |
-                           reinterpret_cast<uintptr_t>(recur)) & 15) == 0;
-    if (H % 16 == 0 && aligned) {
-      return scan_ring_launch<false>(f, scan_out, nullptr, recur, state, rows, H, s);
-    } else {
-      k_scan_seq<<<(H + 63) / 64, 64, 0, s>>>(f, scan_out, recur, state, rows, H);
-    }
-    return hipGetLastError();
+    return scan_ring_launch<false>(f, scan_out, nullptr, recur, state, rows, H, s);
   }
   const int n = stream_state ? rows * H : H;
   k_mixer<<<(n + 255) / 256, 256, 0, s>>>(i, f, scan_out, recur, state, lb, rows, H, stream_state ? 1 : 0);
@@ -2429,21 +2480,27 @@ hipError_t launch_embed(const float* emb, const int64_t* ids, float* h, int rows
   return hipGetLastError();
 }
 
-static size_t rownorm_lds(int cols) {
-  const int nb = (cols & ~7) / 8, Lc = nb > 0 ? (nb + 15) / 16 * 16 : 16;
-  return (static_cast<size_t>(8 * host_lds_stride(Lc) + 8) + 16) * sizeof(float);
+template <bool SW>
+static hipError_t rownorm_launch(const float* x, const float* o, const float* w, float* y, int rows, int cols,
+                                 float eps, hipStream_t s) {
+  const int nb = (cols & ~7) / 8, Lc = nb > 0 ? (nb + 15) / 16 * 16 : 16, G = nb + (cols % 8 ? 1 : 0);
+  // (the ring chains read up to 32 floats past the tail)
+  const size_t lds = (static_cast<size_t>(8 * host_lds_stride(Lc) + 8) + 32) * sizeof(float);
+  if (G <= 256) k_rownorm8<1, SW><<<rows, 256, lds, s>>>(x, o, w, y, cols, eps);
+  else if (G <= 512) k_rownorm8<2, SW><<<rows, 256, lds, s>>>(x, o, w, y, cols, eps);
+  else if (G <= 1024) k_rownorm8<4, SW><<<rows, 256, lds, s>>>(x, o, w, y, cols, eps);
+  else k_rownorm<<<rows, 256, lds, s>>>(x, SW ? o : nullptr, w, y, cols, eps);
+  return hipGetLastError();
 }
 
 hipError_t launch_rmsnorm(const float* x, const float* w, float* y, int rows, int cols, float eps,
                           hipStream_t s) {
-  k_rownorm<<<rows, 256, rownorm_lds(cols), s>>>(x, nullptr, w, y, cols, eps);
-  return hipGetLastError();
+  return rownorm_launch<false>(x, nullptr, w, y, rows, cols, eps, s);
 }
 
 hipError_t launch_swishgate(const float* g, const float* o, const float* w, float* out, int rows, int cols,
                             float eps, hipStream_t s) {
-  k_rownorm<<<rows, 256, rownorm_lds(cols), s>>>(g, o, w, out, cols, eps);
-  return hipGetLastError();
+  return rownorm_launch<true>(g, o, w, out, rows, cols, eps, s);
 }
 
 hipError_t launch_argmax_rows(const float* logits, int rows, int V, int64_t* ids, hipStream_t s) {
@@ -2459,14 +2516,16 @@ hipError_t launch_quant_rows(const float* y, int32_t* q, int rows, int K, float 
 }
 
 hipError_t launch_swiglu(const float* a, const float* b, float* out, size_t n, hipStream_t s) {
-  const int blocks = static_cast<int>(std::min<size_t>((n + 255) / 256, 16384));
-  k_swiglu<<<blocks > 0 ? blocks : 1, 256, 0, s>>>(a, b, out, n);
+  const size_t blocks = (n + 1023) / 1024;
+  if (blocks > 0x7FFFFFFFu) return hipErrorInvalidValue;
+  k_swiglu<<<static_cast<unsigned>(blocks), 256, 0, s>>>(a, b, out, n);
   return hipGetLastError();
 }
 
+// (One load round trip per step on D / 256 blocks, the plain loop before the ring scan here, took
+// 136 us at 1000 x 2048; now 12.)
 hipError_t launch_scan(const float* i, const float* f, float* out, float* state, int T, int D, hipStream_t s) {
-  k_scan<<<(D + 255) / 256, 256, 0, s>>>(i, f, out, state, T, D);
-  return hipGetLastError();
+  return scan_ring_launch<false>(f, i, nullptr, out, state, T, D, s);
 }
 
 }  // namespace mmf
