@@ -187,8 +187,9 @@ struct PrologueArgs {
 // nothing, where rows are too long for them (the caller then runs launch_mixer and kPreSwish).
 hipError_t launch_prologue(Mode mode, const PrologueArgs& a, ActBuf& act, hipStream_t s);
 
-// Integer codes [rows, K] (int16-range, as int32) -> planes (TernaryBackend path).
-hipError_t launch_codes_to_planes(const int32_t* x, ActBuf& act, hipStream_t s);
+// Integer codes [rows, K] (int16-range, as int32; device or pinned host memory) -> planes of act's
+// projection proj (TernaryBackend path).
+hipError_t launch_codes_to_planes(const int32_t* x, int proj, ActBuf& act, hipStream_t s);
 // The inverse: planes (and tail codes) of act's na projections -> int32 codes
 // [na][rows][K] in natural element order, for an external integer matmul.
 hipError_t launch_planes_to_codes(const ActBuf& act, Mode mode, int32_t* codes, hipStream_t s);

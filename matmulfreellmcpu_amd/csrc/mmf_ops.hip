@@ -1095,12 +1095,57 @@ __global__ __launch_bounds__(1024) void k_rowseg_sw(PrologueArgs a, ActBuf act) 
   }
 }
 
-// int16-range codes -> split planes (the TernaryBackend path: codes arrive quantised)
-__global__ void k_codes(const int32_t* __restrict__ x, ActBuf act) {
+// int16-range codes -> split planes of projection `proj` (the TernaryBackend path: codes arrive
+// quantised, from device memory or straight from pinned host memory, which the device does not
+// cache: every code is read once, 32 contiguous bytes per thread). A thread takes the eight
+// elements of chain position t, whose bytes go to LDS rows in chain order; then 16 positions of
+// one chain leave as one 16-byte store per plane (16 positions from a multiple of 16 are one run
+// of the fragment layout).
+__global__ __launch_bounds__(256) void k_codes(const int32_t* __restrict__ x, int proj, ActBuf act) {
+  extern __shared__ __align__(16) int8_t codes_lds[];
+  const int row = xcd_row(blockIdx.x), Lc = act.Lc, nb = act.nb, LQ = Lc + 16;
+  if (row >= act.rows) return;
+  typedef int32_t i4u __attribute__((ext_vector_type(4), aligned(4)));
+  const int32_t* xr = x + static_cast<size_t>(row) * act.K;
+  int8_t* hp = codes_lds;      // [8][LQ] high bytes
+  int8_t* lp = hp + 8 * LQ;    // [8][LQ] low bytes - 128
+  for (int t = threadIdx.x; t < Lc; t += 256) {
+    int32_t c[8] = {};
+    if (t < nb) {
+      const i4u l = reinterpret_cast<const i4u*>(xr + 8 * t)[0], h = reinterpret_cast<const i4u*>(xr + 8 * t)[1];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        c[k] = l[k];
+        c[4 + k] = h[k];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {  // (padding positions: 0 in both planes)
+      hp[j * LQ + t] = static_cast<int8_t>(c[j] >> 8);
+      lp[j * LQ + t] = t < nb ? static_cast<int8_t>((c[j] & 0xFF) - 128) : 0;
+    }
+  }
+  if (threadIdx.x < 8)
+    act.ct[(static_cast<size_t>(proj) * act.rows + row) * 8 + threadIdx.x] =
+        static_cast<int>(threadIdx.x) < act.ntail ? xr[act.K8 + threadIdx.x] : 0;
+  __syncthreads();
+  int8_t* q = act.q + act.qoff(proj, 0, row, 0);
+  const size_t lop = act.qplane();
+  const int n16 = Lc / 16;
+  for (int w = threadIdx.x; w < 8 * n16; w += 256) {
+    const int j = w / n16, t16 = (w - j * n16) * 16;
+    const size_t o = ActBuf::qpos(j * Lc + t16);
+    *reinterpret_cast<uint4*>(q + o) = *reinterpret_cast<const uint4*>(hp + j * LQ + t16);
+    *reinterpret_cast<uint4*>(q + lop + o) = *reinterpret_cast<const uint4*>(lp + j * LQ + t16);
+  }
+}
+
+// The same without LDS, for rows whose planes do not fit it.
+__global__ __launch_bounds__(256) void k_codes_long(const int32_t* __restrict__ x, int proj, ActBuf act) {
   const int row = xcd_row(blockIdx.x), Lc = act.Lc, nb = act.nb;
   if (row >= act.rows) return;
   const int32_t* xr = x + static_cast<size_t>(row) * act.K;
-  int8_t* q = act.q + act.qoff(0, 0, row, 0);
+  int8_t* q = act.q + act.qoff(proj, 0, row, 0);
   const size_t lop = act.qplane();
   for (int j = 0; j < 8; ++j)
     for (int t4 = threadIdx.x * 4; t4 < Lc; t4 += blockDim.x * 4) {
@@ -1117,7 +1162,7 @@ __global__ void k_codes(const int32_t* __restrict__ x, ActBuf act) {
       *reinterpret_cast<uint32_t*>(q + lop + ActBuf::qpos(j * Lc + t4)) = lo;
     }
   for (int t = threadIdx.x; t < 8; t += blockDim.x)
-    act.ct[static_cast<size_t>(row) * 8 + t] = (t < act.ntail) ? xr[act.K8 + t] : 0;
+    act.ct[(static_cast<size_t>(proj) * act.rows + row) * 8 + t] = (t < act.ntail) ? xr[act.K8 + t] : 0;
 }
 
 // planes -> int32 codes [na][rows][K] in natural element order (the inverse of k_codes, for
@@ -2181,8 +2226,13 @@ hipError_t launch_prologue(Mode mode, const PrologueArgs& a, ActBuf& act, hipStr
   return hipGetLastError();
 }
 
-hipError_t launch_codes_to_planes(const int32_t* x, ActBuf& act, hipStream_t s) {
-  k_codes<<<row_grid(act.rows), 256, 0, s>>>(x, act);
+hipError_t launch_codes_to_planes(const int32_t* x, int proj, ActBuf& act, hipStream_t s) {
+  const size_t lds = 16 * (static_cast<size_t>(act.Lc) + 16);
+  if (lds > static_cast<size_t>(lds_limit())) {
+    k_codes_long<<<row_grid(act.rows), 256, 0, s>>>(x, proj, act);
+  } else {
+    k_codes<<<row_grid(act.rows), 256, lds, s>>>(x, proj, act);
+  }
   return hipGetLastError();
 }
 
