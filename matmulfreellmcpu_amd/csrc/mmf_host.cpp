@@ -824,13 +824,14 @@ constexpr size_t kLMFusedMax = 4;
 // width while the row path's hardly grows. Steps of four layers, row path -> fused (us):
 //   integer modes: 1 stream of the 1.3B width FixedQ510 319 -> 161, 8 x 370M 201 -> 188, 10 x 370M
 //   205 -> 204, 3 x 1.3B 266 -> 261, 4 x 1.3B 268 -> 288, 2 x 2.7B 290 -> 278, 3 x 2.7B 296 -> 307;
-//   float: 16 x 370M 310 -> 235, 8 x 1.3B 517 -> 445, 12 x 1.3B 561 -> 592, 6 x 2.7B 605 -> 494.
+//   float: 1 x 370M 159 -> 121, 12 x 370M 220 -> 206, 3 x 1.3B 286 -> 243, 4 x 1.3B 287 -> 303,
+//   2 x 2.7B 274 -> 279, 24 x 370M 246 -> 294.
 // Several streams need H % 8 == 0, so that no element of the gate math over all B * H elements
 // is a SIMD tail element (the row path's rule). The kernels must fit the widths.
 bool step_fused(const Model& m, size_t B) {
   const size_t H = m.cfg.hidden_size;
   const Mode mode = static_cast<Mode>(m.mode);
-  const size_t most = mode == kFloat ? 16384 : (H <= 1024 ? 9216 : 6144);
+  const size_t most = H > 1024 ? 6144 : (mode == kFloat ? 12288 : 9216);
   if (m.ext_on() || (B > 1 && (H % 8 != 0 || B * H > most))) return false;
   for (DecKind k : {kIFG, kO, kGate, kLM})
     if (!decode_fits(k, mode, m.gH)) return false;

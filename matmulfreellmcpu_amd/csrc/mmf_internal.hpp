@@ -224,7 +224,7 @@ hipError_t launch_gemm_mfma(const GemmArgs& a, const ActBuf& act, hipStream_t s)
 // [nmat][rows][N] (integer modes): what the GEMM's epilogue does after its own matmul.
 hipError_t launch_acc_epilogue(const GemmArgs& a, const ActBuf& act, hipStream_t s);
 // Float mode on the fp32 matrix cores (mmf_mfma_f.hip), bit-exact with the FMA chains;
-// used from float_mfma_min_rows() rows on when mfma_f_ok(a).
+// used when mfma_f_ok(a) and the launch has more outputs than the vector-ALU kernel takes.
 bool mfma_f_ok(const GemmArgs& a);
 hipError_t launch_gemm_mfma_f(const GemmArgs& a, const ActBuf& act, hipStream_t s);
 
@@ -257,10 +257,6 @@ size_t gemm_workspace_bytes(const GemmArgs& a);
 // 64 FixedQ510 6.5 -> 6.3; but 3 x 64 x 3000 Int8Absmax 6.9 -> 7.5, 2 x 300 x 6000 8.5 -> 9.1).
 // MMF_MFMA_MIN_ROWS sets another row count (0: never).
 bool int_mfma_rows(Mode mode, int rows, int K);
-// Rows from which float mode uses the fp32 matrix cores (MMF_FLOAT_MFMA_MIN_ROWS, default
-// 16; 0 disables them).
-int float_mfma_min_rows();
-
 // HGRN gate + recurrence over rows (hgrn_model.cpp:109-150). i, f, g: [rows, H].
 // stream_state = false: rows are time steps of one sequence, state [H] carried in order.
 // stream_state = true: rows are independent streams, state [rows, H].

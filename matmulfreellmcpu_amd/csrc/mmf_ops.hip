@@ -17,6 +17,8 @@ namespace mmf {
 
 namespace {
 
+typedef __attribute__((address_space(3))) void lds_void_t;
+
 // Chain-transposed LDS copy of one row for the order-exact row norms: chain j at
 // X[j * LS ...], LS = roundup(Lc, 32) + 4 (the +4 spreads the 8 chain rows over distinct
 // LDS banks), zeros from nb up to roundup(Lc, 32), the tail at X[8 * LS ...].
@@ -1209,40 +1211,26 @@ __global__ __launch_bounds__(kBlock) void k_gemm(GemmArgs a, ActBuf act) {
   slab[0] = P.pk + static_cast<size_t>(og) * g.Wc * 128 + ol * 8 + j;
   if (PAIR) slab[NM - 1] = P.pk + static_cast<size_t>(og + half_groups) * g.Wc * 128 + ol * 8 + j;
 
-  float facc[NM][R];
   int32_t iacc[NM][R], lacc[NM][R];
 #pragma unroll
   for (int mi = 0; mi < NM; ++mi)
 #pragma unroll
-    for (int r = 0; r < R; ++r) { facc[mi][r] = 0.0f; iacc[mi][r] = 0; lacc[mi][r] = 0; }
+    for (int r = 0; r < R; ++r) iacc[mi][r] = lacc[mi][r] = 0;
 
   for (int m0 = 0; m0 < g.Wc; m0 += kMW) {
     const int mw = min(kMW, g.Wc - m0);
     __syncthreads();
     // stage activations [r][chain][mw*16] of this chunk
-    if (MODE == kFloat) {
-      float* L = smem;
-      const int per_row = 8 * mw * 16;
-      for (int e = tid * 4; e < R * per_row; e += kBlock * 4) {
-        const int r = e / per_row, rem = e - r * per_row, jj = rem / (mw * 16), t = rem - jj * mw * 16;
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (r < nrows)
-          v = *reinterpret_cast<const float4*>(
-              act.y + (static_cast<size_t>(ai) * act.rows + row0 + r) * act.ystride() + jj * Lc + m0 * 16 + t);
-        *reinterpret_cast<float4*>(L + r * per_row + jj * mw * 16 + t) = v;
-      }
-    } else {
-      uint32_t* L = reinterpret_cast<uint32_t*>(smem);
-      const int np = (MODE == kFixed) ? 2 : 1;
-      const int per_row = np * 8 * mw * 4;  // dwords
-      for (int e = tid; e < R * per_row; e += kBlock) {
-        const int r = e / per_row, rem = e - r * per_row, pl = rem / (8 * mw * 4),
-                  rem2 = rem - pl * 8 * mw * 4, jj = rem2 / (mw * 4), d = rem2 - jj * mw * 4;
-        uint32_t v = 0;
-        if (r < nrows)
-          v = *reinterpret_cast<const uint32_t*>(act.q + act.qoff(ai, pl, row0 + r, jj * Lc + m0 * 16 + d * 4));
-        L[e] = v;
-      }
+    uint32_t* L = reinterpret_cast<uint32_t*>(smem);
+    constexpr int np = (MODE == kFixed) ? 2 : 1;
+    const int per_row = np * 8 * mw * 4;  // dwords
+    for (int e = tid; e < R * per_row; e += kBlock) {
+      const int r = e / per_row, rem = e - r * per_row, pl = rem / (8 * mw * 4),
+                rem2 = rem - pl * 8 * mw * 4, jj = rem2 / (mw * 4), d = rem2 - jj * mw * 4;
+      uint32_t v = 0;
+      if (r < nrows)
+        v = *reinterpret_cast<const uint32_t*>(act.q + act.qoff(ai, pl, row0 + r, jj * Lc + m0 * 16 + d * 4));
+      L[e] = v;
     }
     __syncthreads();
     for (int mm = 0; mm < mw; ++mm) {
@@ -1250,56 +1238,29 @@ __global__ __launch_bounds__(kBlock) void k_gemm(GemmArgs a, ActBuf act) {
       uint32_t w[NM];
 #pragma unroll
       for (int mi = 0; mi < NM; ++mi) w[mi] = slab[mi][static_cast<size_t>(m) * 128];
-      if (MODE == kFloat) {
-        const float* L = smem;
-        const int per_row = 8 * mw * 16;
-        float wf[NM][16];
+      uint32_t wv[NM][4];
 #pragma unroll
-        for (int mi = 0; mi < NM; ++mi)
+      for (int mi = 0; mi < NM; ++mi)
 #pragma unroll
-          for (int t = 0; t < 16; ++t) wf[mi][t] = code_f(w[mi], t);
+        for (int i = 0; i < 4; ++i) wv[mi][i] = w4_i8(w[mi], i);
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const float* yl = L + r * per_row + j * mw * 16 + mm * 16;
-          float y[16];
+      for (int r = 0; r < R; ++r) {
+        const uint4 h = *reinterpret_cast<const uint4*>(L + r * per_row + j * mw * 4 + mm * 4);
 #pragma unroll
-          for (int q4 = 0; q4 < 4; ++q4) {
-            float4 v = *reinterpret_cast<const float4*>(yl + 4 * q4);
-            y[4 * q4] = v.x; y[4 * q4 + 1] = v.y; y[4 * q4 + 2] = v.z; y[4 * q4 + 3] = v.w;
-          }
-#pragma unroll
-          for (int mi = 0; mi < NM; ++mi)
-#pragma unroll
-            for (int t = 0; t < 16; ++t) facc[mi][r] = __builtin_fmaf(y[t], wf[mi][t], facc[mi][r]);
+        for (int mi = 0; mi < NM; ++mi) {
+          iacc[mi][r] = dot4(wv[mi][0], h.x, iacc[mi][r]);
+          iacc[mi][r] = dot4(wv[mi][1], h.y, iacc[mi][r]);
+          iacc[mi][r] = dot4(wv[mi][2], h.z, iacc[mi][r]);
+          iacc[mi][r] = dot4(wv[mi][3], h.w, iacc[mi][r]);
         }
-      } else {
-        const uint32_t* L = reinterpret_cast<const uint32_t*>(smem);
-        const int np = (MODE == kFixed) ? 2 : 1;
-        const int per_row = np * 8 * mw * 4;
-        uint32_t wv[NM][4];
-#pragma unroll
-        for (int mi = 0; mi < NM; ++mi)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) wv[mi][i] = w4_i8(w[mi], i);
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const uint4 h = *reinterpret_cast<const uint4*>(L + r * per_row + j * mw * 4 + mm * 4);
+        if (MODE == kFixed) {
+          const uint4 l = *reinterpret_cast<const uint4*>(L + r * per_row + 8 * mw * 4 + j * mw * 4 + mm * 4);
 #pragma unroll
           for (int mi = 0; mi < NM; ++mi) {
-            iacc[mi][r] = dot4(wv[mi][0], h.x, iacc[mi][r]);
-            iacc[mi][r] = dot4(wv[mi][1], h.y, iacc[mi][r]);
-            iacc[mi][r] = dot4(wv[mi][2], h.z, iacc[mi][r]);
-            iacc[mi][r] = dot4(wv[mi][3], h.w, iacc[mi][r]);
-          }
-          if (MODE == kFixed) {
-            const uint4 l = *reinterpret_cast<const uint4*>(L + r * per_row + 8 * mw * 4 + j * mw * 4 + mm * 4);
-#pragma unroll
-            for (int mi = 0; mi < NM; ++mi) {
-              lacc[mi][r] = dot4(wv[mi][0], l.x, lacc[mi][r]);
-              lacc[mi][r] = dot4(wv[mi][1], l.y, lacc[mi][r]);
-              lacc[mi][r] = dot4(wv[mi][2], l.z, lacc[mi][r]);
-              lacc[mi][r] = dot4(wv[mi][3], l.w, lacc[mi][r]);
-            }
+            lacc[mi][r] = dot4(wv[mi][0], l.x, lacc[mi][r]);
+            lacc[mi][r] = dot4(wv[mi][1], l.y, lacc[mi][r]);
+            lacc[mi][r] = dot4(wv[mi][2], l.z, lacc[mi][r]);
+            lacc[mi][r] = dot4(wv[mi][3], l.w, lacc[mi][r]);
           }
         }
       }
@@ -1317,19 +1278,7 @@ __global__ __launch_bounds__(kBlock) void k_gemm(GemmArgs a, ActBuf act) {
     for (int mi = 0; mi < NM; ++mi) {
       const int oo = o + (mi ? Nout : 0);
       const size_t ar = static_cast<size_t>(ai) * act.rows + row0 + r;
-      if (MODE == kFloat) {
-        float s = hsum8_lanes(facc[mi][r]);
-        if (j == 0 && r < nrows && oo < g.N) {
-          const float* yt = act.y + ar * act.ystride() + 8 * Lc;
-          for (int t = 0; t < g.ntail; ++t) {
-            const int8_t wt = P.tail[oo * 8 + t];
-            if (wt > 0) s += yt[t];
-            else if (wt < 0) s -= yt[t];
-          }
-        }
-        val[mi] = s * P.inv_scale_w;
-        tot[mi] = 0;
-      } else {
+      {
         int32_t s = isum8_lanes(iacc[mi][r]);
         if (MODE == kFixed) s = s * 256 + isum8_lanes(lacc[mi][r]);
         if (j == 0 && r < nrows && oo < g.N) {
@@ -1363,137 +1312,147 @@ __global__ __launch_bounds__(kBlock) void k_gemm(GemmArgs a, ActBuf act) {
 }
 
 // ------------------------------------------------------------------------------------
-// Float-mode ternary GEMM over row tiles, register-blocked over outputs. Block = 128 threads
-// = 16 output lanes x 8 chains; thread (ol, j) runs chain j (the reference's AVX2 lane j,
-// simd.hpp:92-122: fma(y_k, w_k, a) over k = j + 8t in t order) of NO outputs from NO
-// slabs, for R rows. Activations of kFW words per chain are staged in LDS for the R rows,
-// chain rows padded by 4 floats so the 8 chains of a wave hit distinct banks; each value
-// read feeds NO FMAs and each weight word R x 16. PAIR: the first half of the slabs are
-// gate outputs, the second half their up partners N/2 later (swiglu epilogue).
+// Float-mode ternary GEMM of few rows, on the vector ALUs. Lane (ol, j) of a wave runs chain j
+// (the reference's AVX2 lane j, simd.hpp:92-122: fma(y_k, w_k, a) over k = j + 8t in t order) of
+// NO outputs for R rows; a block's four waves take four neighbouring sets of 8 NO outputs and
+// share the R rows, which move to LDS whole at entry by direct transfers (chain rows 4 floats
+// apart from a multiple of 16, so the 8 chains of a wave read distinct banks). The slab words
+// come four per chain at a time into one of two register sets, the next four in flight. PAIR: NO
+// = 2, a gate output and its up partner N/2 later (swiglu epilogue).
+// Bound by the chain: K / 8 dependent steps of (R NO + decode) instructions per wave, so R and NO
+// (which share LDS reads and weight decodes) grow only while the launch keeps every SIMD four
+// waves (gemm_f_pick). 16 rows, us per BitLinear call against the 16 x 64 matrix-core tiles: see
+// launch_gemm.
 // ------------------------------------------------------------------------------------
-constexpr int kFW = 4;                // words per chain per LDS chunk
-constexpr int kFCS = kFW * 16 + 4;    // floats per staged chain row
+constexpr int kFvWaves = 4;
+
+// floats of one staged row: 8 chain rows and the tail
+__host__ __device__ constexpr int fv_row_floats(int Lc) { return 8 * (Lc + 4) + 8; }
 
 template <int R, int NO, bool PAIR>
-__global__ __launch_bounds__(128) void k_gemm_f(GemmArgs a, ActBuf act) {
-  static_assert(!PAIR || NO % 2 == 0, "gate/up pairs need an even output count");
-  extern __shared__ float smem[];
+__global__ __launch_bounds__(64 * kFvWaves) void k_gemm_f(GemmArgs a, ActBuf act) {
+  static_assert(!PAIR || NO == 2, "a gate output and its up partner");
+  extern __shared__ __align__(16) float smem[];
   const int z = blockIdx.z;
   const ProjDev& P = a.p[z];
-  const Geom& g = P.g;
-  const int Lc = act.Lc, Wc = g.Wc;
-  const int tid = threadIdx.x, ol = tid >> 3, j = tid & 7;
+  const int Lc = act.Lc, Wc = P.g.Wc, N = P.g.N, nt = P.g.ntail, rows = a.rows;
+  const int tid = threadIdx.x, lane = tid & 63, ol = lane >> 3, j = lane & 7;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int row0 = blockIdx.y * R;
-  const int nrows = min(R, a.rows - row0);
   const int am = (act.na > 1) ? z : 0;
-  const int half = g.ngroups / 2;
-  int grp[NO];
-  bool gok[NO];
+  const int Nout = PAIR ? N / 2 : N;
+  const int LS = Lc + 4, RF = fv_row_floats(Lc);
+  // ---- the rows into LDS: float4 p of a row is float4 p % (LS / 4) of chain p / (LS / 4), the
+  // last of each chain padding (any value), then the two of the tail --------------------------
+  {
+    const int c4 = LS / 4, r4 = RF / 4;
+    const uint32_t mc4 = 0xFFFFFFFFu / static_cast<uint32_t>(c4) + 1u;  // p / c4 by a multiply-high
+    const float* yb = act.y + static_cast<size_t>(am) * rows * act.ystride();
+    for (int r = 0; r < R; ++r) {
+      const float* yr = yb + static_cast<size_t>(min(row0 + r, rows - 1)) * act.ystride();
+      for (int p0 = wave * 64; p0 < r4; p0 += 64 * kFvWaves) {
+        const int p = p0 + lane;
+        const int jj = static_cast<int>(__umulhi(static_cast<uint32_t>(p), mc4)), q = p - jj * c4;
+        const float* src = jj < 8 ? yr + jj * Lc + 4 * min(q, c4 - 2) : yr + 8 * Lc + 4 * (q & 1);
+        if (p < r4)
+          __builtin_amdgcn_global_load_lds(src, (lds_void_t*)(smem + r * RF + 4 * p0), 16, 0, 0);
+      }
+    }
+  }
+  // ---- outputs and weights of this wave -------------------------------------------------------
+  const int h0 = blockIdx.x * kFvWaves + wave;  // its set of 8 NO outputs
+  int o[NO];
+  bool ok[NO];
+  const uint32_t* slab[NO];
+  uint2 tw[NO];
+  float addv[NO][R];
 #pragma unroll
   for (int s = 0; s < NO; ++s) {
-    if (PAIR) {
-      const int gg = blockIdx.x * (NO / 2) + (s % (NO / 2));
-      gok[s] = gg < half;
-      grp[s] = (s < NO / 2) ? gg : half + gg;
-    } else {
-      grp[s] = blockIdx.x * NO + s;
-      gok[s] = grp[s] < g.ngroups;
-    }
-    if (!gok[s]) grp[s] = 0;
-  }
-  const uint32_t* slab[NO];
+    const int h = PAIR ? h0 + s * (Nout / 8) : h0 * NO + s;  // half of a 16-output slab group
+    o[s] = 8 * h + ol;
+    ok[s] = PAIR ? 8 * h0 + ol < Nout : o[s] < N;
+    const int hc = min(h, 2 * P.g.ngroups - 1);
+    slab[s] = P.pk + static_cast<size_t>(hc >> 1) * Wc * 128 + (hc & 1) * 64 + lane;
+    const int oc = min(o[s], N - 1);
+    tw[s] = nt ? *reinterpret_cast<const uint2*>(P.tail + 8 * static_cast<size_t>(oc)) : make_uint2(0u, 0u);
 #pragma unroll
-  for (int s = 0; s < NO; ++s) slab[s] = P.pk + static_cast<size_t>(grp[s]) * Wc * 128 + ol * 8 + j;
+    for (int r = 0; r < R; ++r)
+      addv[s][r] = (!PAIR && a.epi == kEpiAdd) ? a.add[static_cast<size_t>(min(row0 + r, rows - 1)) * N + oc] : 0.0f;
+  }
+  constexpr int CW = 4;  // words per chunk
+  uint32_t w[2][CW][NO];
+  auto load = [&](int set, int m0) {
+#pragma unroll
+    for (int u = 0; u < CW; ++u)
+#pragma unroll
+      for (int s = 0; s < NO; ++s) w[set][u][s] = slab[s][static_cast<size_t>(min(m0 + u, Wc - 1)) * 128];
+  };
+  load(0, 0);
   float acc[NO][R];
 #pragma unroll
   for (int s = 0; s < NO; ++s)
 #pragma unroll
     for (int r = 0; r < R; ++r) acc[s][r] = 0.0f;
-  constexpr int PR = 8 * kFCS;  // LDS floats per staged row
-  const float* ybase = act.y + (static_cast<size_t>(am) * act.rows + row0) * act.ystride();
-  for (int m0 = 0; m0 < Wc; m0 += kFW) {
-    const int mw = min(kFW, Wc - m0);
-    uint32_t w[kFW][NO];
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's transfers (and first words) landed
+  __syncthreads();
+  const float* yl = smem + j * LS;
+  auto chunk = [&](int set, int m0) {
 #pragma unroll
-    for (int mm = 0; mm < kFW; ++mm)
+    for (int u = 0; u < CW; ++u) {
+      if (m0 + u >= Wc) break;
 #pragma unroll
-      for (int s = 0; s < NO; ++s)
-        w[mm][s] = (mm < mw && gok[s]) ? slab[s][static_cast<size_t>(m0 + mm) * 128] : 0u;
-    __syncthreads();
-    const int n4 = mw * 4;
-    for (int e = tid; e < R * 8 * n4; e += 128) {
-      const int r = e / (8 * n4), rem = e - r * 8 * n4, jj = rem / n4, q = rem - jj * n4;
-      float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (r < nrows)
-        v = *reinterpret_cast<const float4*>(ybase + static_cast<size_t>(r) * act.ystride() + jj * Lc + m0 * 16 + q * 4);
-      *reinterpret_cast<float4*>(smem + r * PR + jj * kFCS + q * 4) = v;
-    }
-    __syncthreads();
+      for (int i = 0; i < 4; ++i) {  // codes 4i .. 4i + 3 of the word
+        float4 y[R];
 #pragma unroll
-    for (int mm = 0; mm < kFW; ++mm) {
-      if (mm >= mw) break;
-      float wf[NO][16];
+        for (int r = 0; r < R; ++r) y[r] = *reinterpret_cast<const float4*>(yl + r * RF + 16 * (m0 + u) + 4 * i);
 #pragma unroll
-      for (int s = 0; s < NO; ++s)
+        for (int s = 0; s < NO; ++s) {
+          const mmf_half2 e = code_pair_h(w[set][u][s], i, false), d = code_pair_h(w[set][u][s], i, true);
+          const float c0 = static_cast<float>(e.x), c1 = static_cast<float>(d.x), c2 = static_cast<float>(e.y),
+                      c3 = static_cast<float>(d.y);
 #pragma unroll
-        for (int t = 0; t < 16; ++t) wf[s][t] = code_f(w[mm][s], t);
+          for (int r = 0; r < R; ++r) acc[s][r] = __builtin_fmaf(y[r].x, c0, acc[s][r]);
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const float* yl = smem + r * PR + j * kFCS + mm * 16;
-        float y[16];
+          for (int r = 0; r < R; ++r) acc[s][r] = __builtin_fmaf(y[r].y, c1, acc[s][r]);
 #pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) {
-          const float4 v = *reinterpret_cast<const float4*>(yl + 4 * q4);
-          y[4 * q4] = v.x;
-          y[4 * q4 + 1] = v.y;
-          y[4 * q4 + 2] = v.z;
-          y[4 * q4 + 3] = v.w;
+          for (int r = 0; r < R; ++r) acc[s][r] = __builtin_fmaf(y[r].z, c2, acc[s][r]);
+#pragma unroll
+          for (int r = 0; r < R; ++r) acc[s][r] = __builtin_fmaf(y[r].w, c3, acc[s][r]);
         }
-#pragma unroll
-        for (int s = 0; s < NO; ++s)
-#pragma unroll
-          for (int t = 0; t < 16; ++t) acc[s][r] = __builtin_fmaf(y[t], wf[s][t], acc[s][r]);
       }
     }
+  };
+  for (int m0 = 0; m0 < Wc; m0 += 2 * CW) {
+    load(1, m0 + CW);
+    chunk(0, m0);
+    load(0, m0 + 2 * CW);
+    chunk(1, m0 + CW);
   }
-  // reduce the 8 chains of each output (hsum_ps order), tails, scale, epilogue
-  const int Nout = PAIR ? g.N / 2 : g.N;
+  // ---- the 8 chains of each output (hsum_ps order), tails, scale, epilogue ---------------------
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    const size_t ar = static_cast<size_t>(am) * act.rows + row0 + r;
     float val[NO];
 #pragma unroll
     for (int s = 0; s < NO; ++s) {
       float sum = hsum8_lanes(acc[s][r]);
-      const int o = grp[s] * 16 + ol;
-      if (j == 0 && r < nrows && gok[s] && o < g.N) {
-        const float* yt = act.y + ar * act.ystride() + 8 * Lc;
-        for (int t = 0; t < g.ntail; ++t) {
-          const int8_t wt = P.tail[o * 8 + t];
-          if (wt > 0) sum += yt[t];
-          else if (wt < 0) sum -= yt[t];
-        }
+      const float* yt = smem + r * RF + 8 * LS;
+      for (int t = 0; t < nt; ++t) {
+        const int8_t wt = static_cast<int8_t>((t < 4 ? tw[s].x : tw[s].y) >> (8 * (t & 3)));
+        if (wt > 0) sum += yt[t];
+        else if (wt < 0) sum -= yt[t];
       }
       val[s] = sum * P.inv_scale_w;
     }
-    if (j != 0 || r >= nrows) continue;
+    if (j != 0 || row0 + r >= rows) continue;
     const size_t grow = static_cast<size_t>(row0 + r);
     if (PAIR) {
-#pragma unroll
-      for (int s = 0; s < NO / 2; ++s) {
-        const int o = grp[s] * 16 + ol;
-        if (!gok[s] || o >= Nout) continue;
-        const size_t e = grow * Nout + o;
-        a.out[0][e] = swiglu_of(val[s], val[s + NO / 2], static_cast<int64_t>(e) >= (a.swiglu_n & ~7));
-      }
+      if (!ok[0]) continue;
+      const size_t e = grow * Nout + o[0];
+      a.out[0][e] = swiglu_of(val[0], val[NO - 1], static_cast<int64_t>(e) >= (a.swiglu_n & ~7));
     } else {
 #pragma unroll
-      for (int s = 0; s < NO; ++s) {
-        const int o = grp[s] * 16 + ol;
-        if (!gok[s] || o >= g.N) continue;
-        const size_t e = grow * g.N + o;
-        a.out[z][e] = (a.epi == kEpiAdd) ? a.add[e] + val[s] : val[s];
-      }
+      for (int s = 0; s < NO; ++s)
+        if (ok[s]) a.out[z][grow * N + o[s]] = (a.epi == kEpiAdd) ? addv[s][r] + val[s] : val[s];
     }
   }
 }
@@ -1647,8 +1606,6 @@ template <int C>
 constexpr int scan_ring_depth() {
   return C == 4 ? 16 : (C == 8 ? 8 : 4);
 }
-
-typedef __attribute__((address_space(3))) void lds_void_t;
 
 // ANY (a width that is no multiple of C, or rows off 16-byte alignment): transfers of 4 bytes per
 // lane, 64 / C steps x C columns each, columns past the last repeating it (never stored).
@@ -2246,68 +2203,70 @@ template <int MODE, int R, bool PAIR>
 static hipError_t gemm_inst(const GemmArgs& a, const ActBuf& act, hipStream_t s) {
   const Geom& g = a.p[0].g;
   const int np = (MODE == kFixed) ? 2 : 1;
-  const size_t lds = (MODE == kFloat) ? static_cast<size_t>(R) * 8 * kMW * 16 * sizeof(float)
-                                      : static_cast<size_t>(R) * np * 8 * kMW * 16;
+  const size_t lds = static_cast<size_t>(R) * np * 8 * kMW * 16;
   dim3 grid(PAIR ? g.ngroups / 2 : g.ngroups, (a.rows + R - 1) / R, PAIR ? 1 : a.nmat);
   k_gemm<MODE, R, PAIR><<<grid, kBlock, lds, s>>>(a, act);
   return hipGetLastError();
 }
 
-template <int R, int NO, bool PAIR>
-static int gemm_f_blocks(const GemmArgs& a) {
-  const Geom& g = a.p[0].g;
-  const int gx = PAIR ? (g.ngroups / 2 + NO / 2 - 1) / (NO / 2) : (g.ngroups + NO - 1) / NO;
-  return gx * ((a.rows + R - 1) / R) * (PAIR ? 1 : a.nmat);
+// Waves of a k_gemm_f<R, NO> launch.
+static int64_t gemm_f_waves(const GemmArgs& a, int R, int NO) {
+  const bool pair = a.epi == kEpiSwigluPair;
+  const int sets = pair ? a.p[0].g.N / 16 : (a.p[0].g.N + 8 * NO - 1) / (8 * NO);
+  return static_cast<int64_t>(sets) * ((a.rows + R - 1) / R) * (pair ? 1 : a.nmat);
 }
-
 template <int R, int NO, bool PAIR>
 static hipError_t gemm_f_inst(const GemmArgs& a, const ActBuf& act, hipStream_t s) {
-  const Geom& g = a.p[0].g;
-  const size_t lds = static_cast<size_t>(R) * 8 * kFCS * sizeof(float);
-  const int gx = PAIR ? (g.ngroups / 2 + NO / 2 - 1) / (NO / 2) : (g.ngroups + NO - 1) / NO;
-  dim3 grid(gx, (a.rows + R - 1) / R, PAIR ? 1 : a.nmat);
-  k_gemm_f<R, NO, PAIR><<<grid, 128, lds, s>>>(a, act);
+  const int sets = PAIR ? a.p[0].g.N / 16 : (a.p[0].g.N + 8 * NO - 1) / (8 * NO);
+  const dim3 grid((sets + kFvWaves - 1) / kFvWaves, (a.rows + R - 1) / R, PAIR ? 1 : a.nmat);
+  k_gemm_f<R, NO, PAIR><<<grid, 64 * kFvWaves, static_cast<size_t>(R) * fv_row_floats(act.Lc) * sizeof(float), s>>>(a, act);
   return hipGetLastError();
 }
-
-// Four outputs per thread while that leaves at least 1024 blocks (two waves per SIMD),
-// else two, else one: a small launch is latency-bound and wants more waves more than
-// fewer LDS reads.
-template <int R, bool PAIR>
-static hipError_t gemm_f_rows(const GemmArgs& a, const ActBuf& act, hipStream_t s) {
-  if (gemm_f_blocks<R, 4, PAIR>(a) >= 1024) return gemm_f_inst<R, 4, PAIR>(a, act, s);
-  if constexpr (PAIR) {  // a block holds gate/up pairs: at least two outputs per thread
-    return gemm_f_inst<R, 2, PAIR>(a, act, s);
-  } else {
-    if (gemm_f_blocks<R, 2, PAIR>(a) >= 1024) return gemm_f_inst<R, 2, PAIR>(a, act, s);
-    return gemm_f_inst<R, 1, PAIR>(a, act, s);
+// The most outputs per lane that leave four waves per SIMD (a small launch is latency-bound and
+// wants more waves more than fewer LDS reads and decodes); rows of two blocks in a CU's LDS.
+static hipError_t gemm_f_pick(const GemmArgs& a, const ActBuf& act, hipStream_t s) {
+  const size_t row_lds = static_cast<size_t>(fv_row_floats(act.Lc)) * sizeof(float);
+  auto can = [&](int R, int NO) {
+    return a.rows >= R && gemm_f_waves(a, R, NO) >= 4096 && R * row_lds <= 80 * 1024;
+  };
+  if (a.epi == kEpiSwigluPair) {
+    if (can(4, 2)) return gemm_f_inst<4, 2, true>(a, act, s);
+    if (can(2, 2)) return gemm_f_inst<2, 2, true>(a, act, s);
+    return gemm_f_inst<1, 2, true>(a, act, s);
   }
+  if (can(4, 2)) return gemm_f_inst<4, 2, false>(a, act, s);
+  if (can(4, 1)) return gemm_f_inst<4, 1, false>(a, act, s);
+  if (can(2, 2)) return gemm_f_inst<2, 2, false>(a, act, s);
+  if (can(2, 1)) return gemm_f_inst<2, 1, false>(a, act, s);
+  if (can(1, 2)) return gemm_f_inst<1, 2, false>(a, act, s);
+  return gemm_f_inst<1, 1, false>(a, act, s);
+}
+// Float GEMMs of at most kFvOutputs outputs run on the vector ALUs (k_gemm_f): the matrix-core
+// tiles give each SIMD of the chip a chain only from about a hundred 16 x 64 tiles on, and take
+// the same time below. us per BitLinear call, matrix cores (or, up to 15 rows, the FMA kernel
+// before this one) -> vector ALUs: 1 x 1024 x 1024 6.4 -> 5.4, 5 x 2048 x 2048 18.4 -> 8.0, 16 x
+// 2048 x 2048 18.3 -> 10.6, 16 x 5632 x 2048 40.3 -> 21.7, 64 x 1024 x 1024 13.3 -> 10.1, 256 x 300 x
+// 400 11.7 -> 11.5; past it, 96 x 1024 x 1024 13.5 -> 12.0, 24 x 1024 x 5632 13.5 -> 14.6, 48 x
+// 5632 x 2048 43.1 -> 39.6 at 32 rows but 43.9 -> 47.0.
+constexpr int64_t kFvOutputs = 90000;
+
+static bool gemm_f_ok(const GemmArgs& a, const ActBuf& act) {
+  const int64_t outs = static_cast<int64_t>(a.rows) * a.p[0].g.N * (a.epi == kEpiSwigluPair ? 1 : a.nmat);
+  return outs <= kFvOutputs && a.rows <= 65535 && (a.epi != kEpiSwigluPair || a.p[0].g.N % 16 == 0) &&
+         static_cast<size_t>(fv_row_floats(act.Lc)) * sizeof(float) <= static_cast<size_t>(lds_limit());
+}
+
+static hipError_t gemm_float(const GemmArgs& a, const ActBuf& act, hipStream_t s) {
+  if (gemm_f_ok(a, act)) return gemm_f_pick(a, act, s);
+  return mfma_f_ok(a) ? launch_gemm_mfma_f(a, act, s) : hipErrorInvalidValue;
 }
 
 template <int MODE>
 static hipError_t gemm_mode(const GemmArgs& a, const ActBuf& act, hipStream_t s) {
-  if (MODE == kFloat && float_mfma_min_rows() > 0 && a.rows >= float_mfma_min_rows() && mfma_f_ok(a))
-    return launch_gemm_mfma_f(a, act, s);
-  if (MODE == kFloat && a.rows > 4) {
-    const bool pair = a.epi == kEpiSwigluPair;
-    // up to 64 rows (serving steps): 4-row tiles, so that the >= 1024-block rule keeps two
-    // outputs per thread (half the LDS reads per FMA of one) on the 2560-column GEMMs;
-    // 64-stream 2.7B float step 10.9 -> 9.4 ms against 8-row tiles
-    if (a.rows <= 64) return pair ? gemm_f_rows<4, true>(a, act, s) : gemm_f_rows<4, false>(a, act, s);
-    return pair ? gemm_f_rows<16, true>(a, act, s) : gemm_f_rows<16, false>(a, act, s);
-  }
   const bool pair = a.epi == kEpiSwigluPair;
   if (a.rows <= 1) return pair ? gemm_inst<MODE, 1, true>(a, act, s) : gemm_inst<MODE, 1, false>(a, act, s);
   if (a.rows <= 4) return pair ? gemm_inst<MODE, 4, true>(a, act, s) : gemm_inst<MODE, 4, false>(a, act, s);
   return pair ? gemm_inst<MODE, 8, true>(a, act, s) : gemm_inst<MODE, 8, false>(a, act, s);
-}
-
-int float_mfma_min_rows() {
-  static const int v = [] {
-    const char* e = std::getenv("MMF_FLOAT_MFMA_MIN_ROWS");
-    return e ? std::atoi(e) : 16;
-  }();
-  return v;
 }
 
 bool int_mfma_rows(Mode mode, int rows, int K) {
@@ -2329,7 +2288,7 @@ hipError_t launch_gemm(const GemmArgs& a, const ActBuf& act, hipStream_t s) {
     if (ok) return launch_gemm_mfma(a, act, s);
   }
   switch (a.mode) {
-    case kFloat: return gemm_mode<kFloat>(a, act, s);
+    case kFloat: return gemm_float(a, act, s);
     case kFixed: return gemm_mode<kFixed>(a, act, s);
     default: return gemm_mode<kInt8>(a, act, s);
   }
