@@ -282,6 +282,9 @@ hipError_t launch_mixer_segs(const float* i, float* f, float* scan, float* recur
 // rows idx[r] (device) of x [*, K] -> out [n, K]
 hipError_t launch_gather_rows(const float* x, const int* idx, float* out, int n, int K, hipStream_t s);
 
+// n ids from device-readable memory (pinned host memory) to dst.
+hipError_t launch_copy_ids(const int64_t* src, int64_t* dst, int n, hipStream_t s);
+
 // Embedding gather rows (hgrn_model.cpp:321-326).
 hipError_t launch_embed(const float* emb, const int64_t* ids, float* h, int rows, int H,
                         hipStream_t s);

@@ -1811,6 +1811,11 @@ __global__ __launch_bounds__(64 * kScWaves) void k_scan_ring(const float* __rest
   if (wave == 0 && sg == 0 && state && live) state[c0 + cl] = s;
 }
 
+__global__ void k_copy_ids(const int64_t* __restrict__ src, int64_t* __restrict__ dst, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) dst[i] = src[i];
+}
+
 __global__ void k_embed(const float* __restrict__ emb, const int64_t* __restrict__ ids,
                         float* __restrict__ h, int rows, int H) {
   const size_t n = static_cast<size_t>(rows) * H;
@@ -2479,6 +2484,11 @@ hipError_t launch_mixer_segs(const float* i, float* f, float* scan, float* recur
 
 hipError_t launch_gather_rows(const float* x, const int* idx, float* out, int n, int K, hipStream_t s) {
   k_gather_rows<<<n, 256, 0, s>>>(x, idx, out, K);
+  return hipGetLastError();
+}
+
+hipError_t launch_copy_ids(const int64_t* src, int64_t* dst, int n, hipStream_t s) {
+  k_copy_ids<<<(n + 63) / 64, 64, 0, s>>>(src, dst, n);
   return hipGetLastError();
 }
 
