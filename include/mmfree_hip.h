@@ -88,10 +88,10 @@ int mmf_proj_release(mmf_ctx* ctx, int proj_id);
  * stored as int32 (ternary_backend.hpp:8-13). dev pointers. */
 int mmf_ternary_matmul(mmf_ctx* ctx, int proj_id, const int32_t* x, int32_t* acc, size_t b);
 /* The same for k projections on host buffers in one round trip: x[z] holds b rows of K_z
- * codes and acc[z] receives b rows of N_z accumulators for proj_ids[z] (host memory). All
- * codes go to the device in one copy through pinned staging the context keeps, the k matmuls
- * run back to back, and all accumulators return in one copy before the call returns (one
- * synchronisation). TernaryBackend::matmul_batch and matmul_seq (ternary_backend.hpp:43-90)
+ * codes and acc[z] receives b rows of N_z accumulators for proj_ids[z] (host memory). Codes
+ * and accumulators pass through pinned staging the context keeps, which the kernels read and
+ * (up to 8 MB of accumulators) write directly; neighbouring projections of one shape share a
+ * GEMM launch, and the call synchronises once. TernaryBackend::matmul_batch and matmul_seq (ternary_backend.hpp:43-90)
  * on host buffers, as HipTernaryBackend calls it. */
 int mmf_ternary_matmul_host(mmf_ctx* ctx, int k, const int* proj_ids, const int32_t* const* x,
                             int32_t* const* acc, size_t b);
