@@ -453,7 +453,7 @@ def cpu_baselines(blob_dir, ids, gen, gpu_ids):
     allowed cpu. Each dict says what was timed. gpu_ids[(shape, mode)]: the GPU's greedy ids
     for the 16-token prompt, compared with the reference CLI's."""
     if not os.path.exists(REF_CLI):
-        return None, None, {}, None
+        return None, {}, None
     sock, allc = cpu_sets()
     env_s, env_a = omp_env(sock), omp_env(allc)
     res = {}
