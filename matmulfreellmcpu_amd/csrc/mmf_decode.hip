@@ -17,11 +17,14 @@
 //    words per matrix, the epilogue operands, the prologue inputs -- is issued at entry;
 //  * every block recomputes the (order-exact) row norms of its input vector, so no
 //    grid-wide synchronisation is needed inside a launch.
+// ST (a serving step of few streams): blockIdx.y is the stream, whose vectors, state, token, logits
+// and keys follow the first stream's.
 // Thread (ol, j) of a matrix's 128 threads sums chain j of output og*16+ol, which is the
 // reference's AVX2 lane j (16 outputs x 8 chains per output group).
 #include <hip/hip_ext.h>
 
 #include <cstdlib>
+#include <type_traits>
 
 #include "mmf_device.hpp"
 #include "mmf_internal.hpp"
@@ -91,7 +94,7 @@ __device__ __forceinline__ void load_seg(const float* p, int l, float4 (&d)[RC],
 template <int MODE, int KIND, int RC>
 constexpr int kDecMinWaves = (MODE != kFloat && KIND == kGate && RC > 0) ? 4 : 1;
 
-template <int MODE, int KIND, int NV, int KS, int RC, bool W4>
+template <int MODE, int KIND, int NV, int KS, int RC, bool W4, bool ST>
 __global__ __launch_bounds__(kBlock * KindTraits<KIND>::NM * KS) __attribute__((amdgpu_waves_per_eu(kDecMinWaves<MODE, KIND, RC>)))
 void k_decode(DecArgs a) {
   static_assert(!W4 || (MODE == kFloat && KIND != kLM), "fp4 words are for the float layer GEMVs");
@@ -151,20 +154,26 @@ void k_decode(DecArgs a) {
 #undef MMF_PIN_BASE
   const int Ww = W4 ? 2 * Wc : Wc;  // slab words per chain
   const int W = 8 * Lc + 8;  // floats of a chain-transposed vector in global memory
-  const int sb = blockIdx.y;  // the stream: its vectors follow the first stream's
-  if (sb > 0) {
+  const int sb = ST ? blockIdx.y : 0;  // the stream: its vectors follow the first stream's
+  if constexpr (ST) {
     const size_t oi = static_cast<size_t>(sb) * W, oo = static_cast<size_t>(sb) * (8 * aoLc + 8);
-    if (ax) ax += oi;
-    if (KIND == kO) ax2 += oi;
-    if (KIND == kO || KIND == kDown) ahin += oo;
-    if (KIND == kIFG) {
+    if constexpr (KIND == kIFG) ax = ax ? ax + oi : nullptr;
+    else ax += oi;
+    if constexpr (KIND == kO) ax2 += oi;
+    if constexpr (KIND == kO || KIND == kDown) ahin += oo;
+    if constexpr (KIND == kIFG) {
       astate += static_cast<size_t>(sb) * aH;
       arecur += oo;
       agout += oo;
+      aout = aout ? aout + oo : nullptr;
+    } else if constexpr (KIND == kLM) {
+      aout = aout ? aout + static_cast<size_t>(sb) * avocab : nullptr;
+      akeys = akeys ? akeys + static_cast<size_t>(sb) * kLMBlocks : nullptr;
+    } else if constexpr (KIND == kDown) {
+      aout += a.out_nat ? static_cast<size_t>(sb) * gN : oo;
+    } else {
+      aout += oo;
     }
-    if (aout) aout += (KIND == kLM) ? static_cast<size_t>(sb) * avocab
-                      : (KIND == kDown && a.out_nat) ? static_cast<size_t>(sb) * gN : oo;
-    if (KIND == kLM && akeys) akeys += static_cast<size_t>(sb) * kLMBlocks;
   }
   const int F4 = W / 4;  // float4s of a chain-transposed vector
   // LDS copies pad each chain row by 16 bytes so that the 8 chain lanes of a wave read
@@ -210,7 +219,7 @@ void k_decode(DecArgs a) {
 
   // layer 0: the token is the argmax over the previous lm_head's per-block keys
   int64_t tok = 0;
-  if (KIND == kIFG && ax == nullptr && a.tokens) {
+  if (ST && KIND == kIFG && ax == nullptr) {
     tok = a.tokens[sb];
   } else if (KIND == kIFG && ax == nullptr) {
     unsigned long long best = 0ull;
@@ -673,7 +682,7 @@ void k_decode(DecArgs a) {
       agout[p] = v2;
       if (aout) aout[p] = src[0][p];  // layer 0: the embedding row becomes h
     } else if (KIND == kO || KIND == kDown) {
-      aout[(KIND == kDown && a.out_nat) ? o : p] = e_hin + val;
+      aout[(ST && KIND == kDown && a.out_nat) ? o : p] = e_hin + val;
     } else {  // kGate
       aout[p] = swiglu_of(val, v1, o >= (nout & ~7));
     }
@@ -712,7 +721,7 @@ struct DecfShape {
   static constexpr int SLICE = ACT + NW * 64 + TR;  // + the wave's words (+ the staging)
 };
 
-template <int MODE, int KIND, int RC>
+template <int MODE, int KIND, int RC, bool ST>
 __global__ __launch_bounds__(64 * KindTraits<KIND>::NM) void k_decf(const float* __restrict__ xin,
                                                                    const float* __restrict__ prew,
                                                                    const float* __restrict__ xg,
@@ -741,12 +750,12 @@ __global__ __launch_bounds__(64 * KindTraits<KIND>::NM) void k_decf(const float*
   const float aeps = a.eps;
   const int nout = gN;
   constexpr int W = 8 * S::Lc + 8;
-  const int sb = blockIdx.y;  // the stream: its input vectors follow the first stream's
+  const int sb = ST ? blockIdx.y : 0;  // the stream: its input vectors follow the first stream's
 
   // layer 0: the token is the argmax over the previous lm_head's per-block keys (every wave
   // reduces all keys itself), or the caller's
-  const float* src0 = xin + static_cast<size_t>(sb) * W;
-  if (KIND == kIFG && xin == nullptr && a.tokens) {
+  const float* src0 = ST ? xin + static_cast<size_t>(sb) * W : xin;
+  if (ST && KIND == kIFG && xin == nullptr) {
     src0 = a.embT + static_cast<size_t>(a.tokens[sb]) * W;
   } else if (KIND == kIFG && xin == nullptr) {
     const unsigned long long* keys = a.keys;
@@ -829,8 +838,8 @@ __global__ __launch_bounds__(64 * KindTraits<KIND>::NM) void k_decf(const float*
   const bool epi = mi == 0 && j == 0 && o < nout;
   const int po = epi ? (KIND == kOp ? o : ((o < a.oK8) ? (o & 7) * a.oLc + (o >> 3) : 8 * a.oLc + (o - a.oK8))) : 0;
   // this stream's outputs (kIFG: state and the H-long vectors; kO, kDown: one vector)
-  const size_t so = static_cast<size_t>(sb) * (8 * a.oLc + 8);
-  const bool nat = KIND == kDown && a.out_nat;
+  const size_t so = ST ? static_cast<size_t>(sb) * (8 * a.oLc + 8) : 0;
+  const bool nat = ST && KIND == kDown && a.out_nat;
   float* const state_b = (KIND == kIFG) ? a.state + static_cast<size_t>(sb) * a.H : nullptr;
   float* const out_b = (KIND == kOp || (KIND == kIFG && !a.out)) ? a.out : a.out + (nat ? static_cast<size_t>(sb) * gN : so);
   float e_lb = 0.0f, e_st = 0.0f, e_hin = 0.0f;
@@ -1063,6 +1072,12 @@ __global__ __launch_bounds__(64 * KindTraits<KIND>::NM) void k_decf(const float*
   }
 }
 
+// Whether a launch is one of a serving step (the kernels' ST form: the caller's tokens, streams in
+// blockIdx.y). The batch-1 decode keeps kernels without it: with stream offsets in them its i/f/g
+// launch took 8.58 us against 8.32 (2560 wide, FixedQ510) and 8.02 against 7.76 (float), the
+// lm_head 11.54 against 11.46; a 12-layer float step 444.5 against 437.3.
+bool is_step(const DecArgs& a) { return a.streams > 0; }
+
 template <int MODE, int KIND, int RC>
 hipError_t decf_rc(const DecArgs& a, hipStream_t s) {
   using S = DecfShape<MODE, KIND, RC>;
@@ -1070,8 +1085,13 @@ hipError_t decf_rc(const DecArgs& a, hipStream_t s) {
   const dim3 grid((a.p[0].g.N + 7) / 8, a.streams > 1 ? a.streams : 1);
   const float* prew = (KIND == kDown || KIND == kOp) ? nullptr : a.pre_w;
   const float* xg = (KIND == kO) ? a.x2 : nullptr;
-  return launch_k(k_decf<MODE, KIND, RC>, grid, 64 * S::NM, lds, s, a.x, prew, xg, a.p[0].normwT, a.p[1].normwT,
-                  a.p[2].normwT, a);
+  auto go = [&](auto k) {
+    return launch_k(k, grid, 64 * S::NM, lds, s, a.x, prew, xg, a.p[0].normwT, a.p[1].normwT, a.p[2].normwT, a);
+  };
+  if constexpr (KIND != kOp) {
+    if (is_step(a)) return go(k_decf<MODE, KIND, RC, true>);
+  }
+  return go(k_decf<MODE, KIND, RC, false>);
 }
 
 // k_decf for a layer kind when every matrix has its slab (float: the fp4 one) and a chain-
@@ -1144,7 +1164,8 @@ hipError_t dec_rc(const DecArgs& a, size_t lds, dim3 grid, hipStream_t s) {
   constexpr int BS = kBlock * KindTraits<KIND>::NM * KS;
   constexpr int F4 = (8 * 32 * RC + 8) / 4;  // float4s of a chain-transposed vector
   static_assert(F4 <= 16 * BS, "row too long for the block layout");
-  return launch_k(k_decode<MODE, KIND, nv_for(F4, BS), KS, RC, W4>, grid, BS, lds, s, a);
+  if (is_step(a)) return launch_k(k_decode<MODE, KIND, nv_for(F4, BS), KS, RC, W4, true>, grid, BS, lds, s, a);
+  return launch_k(k_decode<MODE, KIND, nv_for(F4, BS), KS, RC, W4, false>, grid, BS, lds, s, a);
 }
 
 template <int MODE, int KIND, int KS, bool W4>
@@ -1169,10 +1190,15 @@ hipError_t dec_ks(const DecArgs& a, size_t lds, dim3 grid, hipStream_t s) {
     }
   }
   const int F4 = (8 * Lc + 8) / 4;
-  if (F4 <= 2 * BS) return launch_k(k_decode<MODE, KIND, 2, KS, 0, W4>, grid, BS, lds, s, a);
-  if (F4 <= 4 * BS) return launch_k(k_decode<MODE, KIND, 4, KS, 0, W4>, grid, BS, lds, s, a);
-  if (F4 <= 8 * BS) return launch_k(k_decode<MODE, KIND, 8, KS, 0, W4>, grid, BS, lds, s, a);
-  if (F4 <= 16 * BS) return launch_k(k_decode<MODE, KIND, 16, KS, 0, W4>, grid, BS, lds, s, a);
+  auto go = [&](auto nv) {
+    constexpr int NV = decltype(nv)::value;
+    if (is_step(a)) return launch_k(k_decode<MODE, KIND, NV, KS, 0, W4, true>, grid, BS, lds, s, a);
+    return launch_k(k_decode<MODE, KIND, NV, KS, 0, W4, false>, grid, BS, lds, s, a);
+  };
+  if (F4 <= 2 * BS) return go(std::integral_constant<int, 2>{});
+  if (F4 <= 4 * BS) return go(std::integral_constant<int, 4>{});
+  if (F4 <= 8 * BS) return go(std::integral_constant<int, 8>{});
+  if (F4 <= 16 * BS) return go(std::integral_constant<int, 16>{});
   return hipErrorInvalidValue;
 }
 
