@@ -135,7 +135,8 @@ int mmf_swiglu(mmf_ctx* ctx, float* out, const float* a, const float* b, size_t 
 /* hgrn_scan (kernels.hpp:55-59, hgrn_scan.cpp:11-19): state may be NULL (zeros) */
 int mmf_hgrn_scan(mmf_ctx* ctx, float* out, const float* i, const float* f, size_t T, size_t D,
                   float* state);
-/* rmsnorm_swishgate (kernels.hpp:61-63, rmsnorm_swishgate.cpp:13-30) */
+/* rmsnorm_swishgate (kernels.hpp:61-63, rmsnorm_swishgate.cpp:13-30); o may be NULL (no gate:
+ * the plain rmsnorm of g) */
 int mmf_rmsnorm_swishgate(mmf_ctx* ctx, float* out, const float* g, const float* o,
                           const float* w, size_t rows, size_t cols, float eps);
 

@@ -2519,6 +2519,8 @@ hipError_t launch_rmsnorm(const float* x, const float* w, float* y, int rows, in
 
 hipError_t launch_swishgate(const float* g, const float* o, const float* w, float* out, int rows, int cols,
                             float eps, hipStream_t s) {
+  // (no gate rows: the plain norm)
+  if (!o) return rownorm_launch<false>(g, nullptr, w, out, rows, cols, eps, s);
   return rownorm_launch<true>(g, o, w, out, rows, cols, eps, s);
 }
 

@@ -40,6 +40,19 @@ def test_norms(eng, oracle, cols):  # noqa: F811
         assert_bitexact(kx.get()[off:].reshape(rows, cols), oracle.rmsnorm(x, w, 1e-6), "rmsnorm in place")
 
 
+@pytest.mark.parametrize("cols", [7, 100, 2049, 9000])
+def test_swishgate_without_gate(eng, oracle, cols):  # noqa: F811
+    """A null gate is the plain norm, on the short-row kernel as on the long-row one."""
+    print(f"swishgate without gate cols={cols}", flush=True)
+    rng = np.random.default_rng(cols)
+    x = rng.standard_normal((3, cols)).astype(np.float32)
+    w = (1 + 0.1 * rng.standard_normal(cols)).astype(np.float32)
+    dx, dw, y = Dev(eng, x), Dev(eng, w), Dev(eng, shape=(3, cols))
+    eng.rmsnorm_swishgate(y.ptr, dx.ptr, None, dw.ptr, 3, cols)
+    eng.sync()
+    assert_bitexact(y.get(), oracle.rmsnorm(x, w, 1e-6), "norm")
+
+
 @pytest.mark.parametrize("n", [1, 7, 8, 12, 1023, 1024, 1029, 100003])
 def test_swiglu_sizes(eng, oracle, n):  # noqa: F811
     rng = np.random.default_rng(n)
