@@ -1982,14 +1982,15 @@ __global__ void k_quant_rows(const float* __restrict__ y, int32_t* __restrict__ 
 // Four elements per thread (16-byte accesses, at any 4-byte alignment); bound by memory.
 __global__ __launch_bounds__(256) void k_swiglu(const float* __restrict__ a, const float* __restrict__ b,
                                                 float* __restrict__ out, size_t n) {
-  const size_t body = n & ~static_cast<size_t>(7);
-  const size_t e = 4 * (blockIdx.x * static_cast<size_t>(256) + threadIdx.x);
-  if (e < body) {  // (body is a multiple of 4)
-    const f4u x = *reinterpret_cast<const f4u*>(a + e), y = *reinterpret_cast<const f4u*>(b + e);
-    *reinterpret_cast<f4u*>(out + e) = f4u{swiglu_of(x[0], y[0], false), swiglu_of(x[1], y[1], false),
-                                           swiglu_of(x[2], y[2], false), swiglu_of(x[3], y[3], false)};
-  } else {
-    for (size_t k = e; k < n && k < e + 4; ++k) out[k] = swiglu_of(a[k], b[k], true);
+  const size_t body = n & ~static_cast<size_t>(7), step = static_cast<size_t>(gridDim.x) * 1024;
+  for (size_t e = 4 * (blockIdx.x * static_cast<size_t>(256) + threadIdx.x); e < n; e += step) {
+    if (e < body) {  // (body is a multiple of 4)
+      const f4u x = *reinterpret_cast<const f4u*>(a + e), y = *reinterpret_cast<const f4u*>(b + e);
+      *reinterpret_cast<f4u*>(out + e) = f4u{swiglu_of(x[0], y[0], false), swiglu_of(x[1], y[1], false),
+                                             swiglu_of(x[2], y[2], false), swiglu_of(x[3], y[3], false)};
+    } else {
+      for (size_t k = e; k < n && k < e + 4; ++k) out[k] = swiglu_of(a[k], b[k], true);
+    }
   }
 }
 
@@ -2537,8 +2538,8 @@ hipError_t launch_quant_rows(const float* y, int32_t* q, int rows, int K, float 
 }
 
 hipError_t launch_swiglu(const float* a, const float* b, float* out, size_t n, hipStream_t s) {
-  const size_t blocks = (n + 1023) / 1024;
-  if (blocks > 0x7FFFFFFFu) return hipErrorInvalidValue;
+  // (a launch holds fewer than 2^32 threads; the kernel's loop takes what is beyond 2^20 blocks)
+  const size_t blocks = std::min<size_t>((n + 1023) / 1024, 1u << 20);
   k_swiglu<<<static_cast<unsigned>(blocks), 256, 0, s>>>(a, b, out, n);
   return hipGetLastError();
 }

@@ -65,6 +65,29 @@ def test_swiglu_sizes(eng, oracle, n):  # noqa: F811
         assert_bitexact(out.get()[off:], oracle.swiglu(a, b), f"swiglu n={n}")
 
 
+def test_swiglu_beyond_a_grid(eng, oracle):  # noqa: F811
+    """More elements than 2^32 threads of four (64 GiB, in place): some at the start, past 2^32
+    elements, past 2^30 (the largest grid's first sweep) and the tail."""
+    n = (1 << 34) + 13
+    print(f"swiglu n={n}", flush=True)
+    big = Dev(eng, shape=(n,))
+    rng = np.random.default_rng(5)
+    at = {e: rng.standard_normal(13).astype(np.float32) * 4 for e in (0, (1 << 30) - 5, (1 << 32) + 7, (1 << 34) - 40, n - 13)}
+    for e, v in at.items():
+        eng._chk(eng.lib.mmf_upload(eng.h, big.ptr + 4 * e, v.ctypes.data, v.nbytes))
+    eng.swiglu(big.ptr, big.ptr, big.ptr, n)
+    eng.sync()
+    for e, v in at.items():
+        got = np.empty_like(v)
+        eng._chk(eng.lib.mmf_download(eng.h, got.ctypes.data, big.ptr + 4 * e, got.nbytes))
+        tail = 5 if e == n - 13 else 0  # n % 8 elements go by the tail rule
+        pad = np.concatenate([v[:13 - tail], np.zeros(3 + tail, np.float32)])  # (a multiple of 8: no tail)
+        want = oracle.swiglu(pad, pad)[:13 - tail]
+        if tail:
+            want = np.concatenate([want, oracle.swiglu(v[-tail:], v[-tail:])])
+        assert_bitexact(got, want, f"swiglu at {e}")
+
+
 # the ring scan (16-byte transfers at D % 8 == 0, aligned; else 4-byte ones) over less than, exactly and more than whole 128-step tiles,
 # and partial column groups
 @pytest.mark.parametrize("T,D,off", [(1, 16, 0), (5, 2048, 0), (127, 64, 0), (128, 64, 0), (129, 48, 0), (1000, 256, 0),
