@@ -42,9 +42,10 @@
 // waves per SIMD with the same tile traffic and no partials through memory: eight one-wave
 // groups carry every launch of up to a few hundred small tiles, two groups the 128 x 128 tiles
 // at one block per CU.
-// Split-K (K beyond 6912 with few tiles): blockIdx.y selects a contiguous range of stages; each
-// block stores its exact int32 partial tile, and k_splitk_epi adds the partials in split order
-// and applies the epilogue (integer sums: the order does not change the result).
+// Split-K (K beyond 13824, or beyond 9216 with a handful of tiles; plan_of): blockIdx.y selects a
+// contiguous range of stages; each block stores its exact int32 partial tile, and k_splitk_epi
+// adds the partials in split order and applies the epilogue (integer sums: the order does not
+// change the result).
 #include <cstdlib>
 #include <type_traits>
 
@@ -919,20 +920,27 @@ bool mfma_launch(const GemmArgs& a, const ActBuf& act, dim3 grid, hipStream_t s)
 // limits 512 x 513 x 5000 FixedQ510 17.1 -> 20.9 (64 x 64), 384 x 1024 x 5632 Int8Absmax 14.4 ->
 // 17.4 (32 x 64). Below K = 512 the second round does not pay (384 x 64 x 3000: 10.9 -> 11.9).
 // Above that: 128-row tiles (64 rows for the few-row launches of very wide matrices), 256
-// columns when that still gives every CU a block (all blocks of all matrices), else 128. For K
-// beyond 6912 (stages beyond kGroupStages), K is split in powers of two until there are 128
-// blocks (each split >= 4 stages): the eight waves of one block would walk too many stages.
+// columns when that still gives every CU a block (all blocks of all matrices), else 128.
+// K is split in powers of two until there are 128 blocks (each split >= 4 stages) where the eight
+// waves of one block would walk too many stages: beyond kGroupStages stages of 64 elements (K
+// 13824), and beyond kFewStages (K 9216) for at most 40 rows of at most eight 64 x 128 tiles, whose
+// 16 splits have 32 waves where a K-group tile has eight (us per call, K-groups -> split: 8 x 12288
+// x 256 FixedQ510 24.2 -> 23.1, Int8Absmax 22.8 -> 21.2, 8 x 13824 x 1024 27.0 -> 25.0 and 25.1 ->
+// 22.6; but 32 x 8836 x 1024 21.7 -> 22.8 and 20.3 -> 21.1, at 64 rows 12288 x 1024 25.0 -> 26.7 and
+// 23.4 -> 24.0, at 16 tiles, 8 x 13824 x 2048, 27.0 -> 29.1 and 25.3 -> 25.1). Between the two limits
+// everything else keeps the K-groups: 100 x 13824 x 4096 32.6 -> 48.9, 16 x 12288 x 4096 25.1 -> 37.8.
 struct Plan {
   int wm, wn, ksplit, kw;
   int fm = 2;  // 32-row fragments per wave (1: 32-row tiles)
 };
-constexpr int kGroupStages = 216;
+constexpr int kGroupStages = 216, kFewStages = 144;
 
 Plan plan_of(const GemmArgs& a) {
   const int nz = (a.epi == kEpiSwigluPair) ? 1 : a.nmat;
   const int nst = a.p[0].g.Lc / 8;
   const int t32 = tiles_of<1, 1, 1>(a) * nz, t64 = tiles_of<1, 1>(a) * nz;
-  if (nst <= kGroupStages) {
+  const bool split = nst > kGroupStages || (nst > kFewStages && a.rows <= 40 && tiles_of<1, 2>(a) * nz <= 8);
+  if (!split) {
     const bool two = a.p[0].g.K >= 512;  // a second round of tiles
     if (t32 <= 256) return Plan{1, 1, 1, 8, 1};
     if (t64 <= 256 || (two && a.mode == kFixed && t64 <= 512)) return Plan{1, 1, 1, 8, 2};
@@ -957,7 +965,7 @@ Plan plan_of(const GemmArgs& a) {
                                : (p.wn == 4 ? tiles_of<2, 4>(a) : tiles_of<2, 2>(a))) * nz;
   // split K until there are 128 blocks (one per two CUs; more splits measured slower, the
   // partial traffic growing with the split count), keeping >= 4 stages per split
-  if (nst > kGroupStages)
+  if (split)
     while (tiles * p.ksplit < 128 && nst / (2 * p.ksplit) >= 4 && p.ksplit < 16) p.ksplit *= 2;
   // 128 x 128 tiles at one block per CU (the 2048-column o/down GEMMs of a long prefill):
   // two K-groups per block give each SIMD two waves instead of one, with the same tile

@@ -43,6 +43,52 @@ def test_bitlinear_odd(eng, oracle, rows, K, N, mode):  # noqa: F811
     eng.proj_release(pid)
 
 
+# (rows, K, N) around the plan's limits on splitting K: 144 stages of 64 elements (K 9216, then
+# chains in steps of 16 positions) with at most 40 rows of eight 64 x 128 tiles, and 216 stages (K
+# 13824) whatever the tiles; partial tiles, tails, and the 64- and 128-row tiles split
+SPLIT = [(2, 9223, 70), (3, 9224, 70), (40, 9230, 1024), (41, 9230, 1024), (17, 9345, 1025), (40, 13831, 40),
+         (5, 13832, 40), (40, 14003, 333), (100, 16384, 64), (200, 13900, 700)]
+
+
+@pytest.mark.parametrize("mode", [FIXED, INT8])
+@pytest.mark.parametrize("rows,K,N", SPLIT)
+def test_bitlinear_split_k(eng, oracle, rows, K, N, mode):  # noqa: F811
+    """Long rows whose K is split over blocks: outputs and accumulators, through the context's
+    workspace and, with a smaller second call on what the first left, the static scratch."""
+    print(f"split rows={rows} K={K} N={N} mode={mode}", flush=True)
+    rng = np.random.default_rng(rows + K + N + mode)
+    x = (rng.standard_normal((rows, K)) * 2).astype(np.float32)
+    nw = (1 + 0.1 * rng.standard_normal(K)).astype(np.float32)
+    wq = rng.integers(-1, 2, (N, K)).astype(np.int8)
+    sw = float(np.float32(1.0 / 0.0157))
+    want = oracle.bitlinear(x, nw, wq, sw, 1e-6, mode)
+    pid = eng.register_proj(wq, sw, nw)
+    dx, dout, dacc = Dev(eng, x), Dev(eng, shape=(rows, N)), Dev(eng, shape=(rows, N), dtype=np.int32)
+    for fn in (eng.bitlinear, eng.bitlinear_noalloc):
+        for n in (rows, max(2, rows // 2)):
+            for acc in (dacc.ptr, None):
+                fn(pid, dx.ptr, dout.ptr, n, mode=mode, acc=acc)
+                eng.sync()
+                assert_bitexact(dout.get()[:n], want["out"][:n], f"out of {n} rows")
+            np.testing.assert_array_equal(dacc.get()[:n], want["acc"][:n])
+    eng.proj_release(pid)
+
+
+@pytest.mark.parametrize("mode", [FIXED, INT8])
+@pytest.mark.parametrize("hidden,inter,layers", [(16, 9232, 2), (9232, 32, 1)])
+def test_model_split_k(tmp_path, oracle, hidden, inter, layers, mode):
+    """Prompts whose residual or whose swiglu-pair GEMM splits K: logits of every position."""
+    from matmulfreellmcpu_amd import Engine, make_blob, read_blob
+    print(f"split model hidden={hidden} mode={mode}", flush=True)
+    blob = read_blob(make_blob(str(tmp_path / "m"), vocab=200, hidden=hidden, layers=layers, inter=inter, seed=5,
+                               random_norms=True, random_lb=True))
+    ids = np.random.default_rng(2).integers(0, 200, 6)
+    e = Engine(0)
+    e.load_blob(blob, mode)
+    assert_bitexact(e.forward(ids), oracle.model(blob).forward(ids, mode), "logits")
+    e.close()
+
+
 @pytest.mark.parametrize("hidden", [100, 250, 1027])
 @pytest.mark.parametrize("mode", [FLOAT, FIXED, INT8])
 def test_serve_odd_hidden(tmp_path, oracle, hidden, mode):
