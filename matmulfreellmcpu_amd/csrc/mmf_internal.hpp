@@ -251,12 +251,19 @@ hipError_t measure_peaks(int cus, hipStream_t s, double out[4]);
 // Bytes of int32 workspace launch_gemm needs for `a` (0 when it will not split K); the
 // caller passes at least that much in a.ws.
 size_t gemm_workspace_bytes(const GemmArgs& a);
-// Whether the integer modes run a GEMM of these rows over K on the matrix cores: from 3 (FixedQ510)
-// or 4 rows, and below where rows * K >= 1024 (us per BitLinear call, dot products -> matrix
-// cores: 2 x 1024 x 5632 FixedQ510 11.3 -> 7.1, Int8Absmax 8.2 -> 7.1, 7 rows 21.8 -> 7.3, 3 x 64 x
-// 64 FixedQ510 6.5 -> 6.3; but 3 x 64 x 3000 Int8Absmax 6.9 -> 7.5, 2 x 300 x 6000 8.5 -> 9.1).
+// Whether an integer-mode GEMM runs on the matrix cores. They take 32 rows for one, so few rows pay
+// where K is long against the tile's fixed cost, and one row only while its 32 x 64 tiles fit one
+// round (us per call, dot products -> matrix cores; 5 rows and more: always).
+//   1 row: FixedQ510 from K 1024, Int8Absmax from 2560, up to 16384 outputs (Int8Absmax from K 4096
+//     on 49152; 8192 beyond K 13824, where the tiles split K): 4096 x 5632 FixedQ510 17.4 -> 13.0,
+//     9000 x 32000 Int8Absmax 36.4 -> 27.4; but 1024 x 16896 FixedQ510 9.3 -> 13.7, 7396 x 60675 64 ->
+//     78, 2048 x 7116 Int8Absmax 9.6 -> 9.8.
+//   2 - 4 rows: rows * K >= 1024 (FixedQ510: 3 rows from K 256, 4 rows always, 2 rows below K 1024 to
+//     16384 outputs only; Int8Absmax: 2 rows from K 1024): 2 x 1024 x 5632 FixedQ510 12.4 -> 8.1; but 2 x 512 x
+//     16896 11.4 -> 12.4, 3 x 64 x 20225 8.5 -> 9.1, 4 x 64 x 256 Int8Absmax 8.1 -> 8.3. Or 49152
+//     outputs: 3 x 64 x 100000 FixedQ510 14.0 -> 9.8; but 2 x 64 x 33792 9.3 -> 9.8.
 // MMF_MFMA_MIN_ROWS sets another row count (0: never).
-bool int_mfma_rows(Mode mode, int rows, int K);
+bool int_mfma_rows(const GemmArgs& a);
 // HGRN gate + recurrence over rows (hgrn_model.cpp:109-150). i, f, g: [rows, H].
 // stream_state = false: rows are time steps of one sequence, state [H] carried in order.
 // stream_state = true: rows are independent streams, state [rows, H].

@@ -1039,7 +1039,7 @@ hipError_t launch_pack_mfma(const uint32_t* pk, const Geom& g, bool pair, uint32
 }
 
 size_t gemm_workspace_bytes(const GemmArgs& a) {
-  if (a.mode == kFloat || !int_mfma_rows(a.mode, a.rows, a.p[0].g.K)) return 0;
+  if (a.mode == kFloat || !int_mfma_rows(a)) return 0;
   const Plan p = plan_of(a);
   if (p.ksplit == 1) return 0;
   return static_cast<size_t>(p.ksplit) * a.nmat * a.rows * static_cast<size_t>(a.p[0].g.N) * sizeof(int32_t);

@@ -2275,17 +2275,26 @@ static hipError_t gemm_mode(const GemmArgs& a, const ActBuf& act, hipStream_t s)
   return pair ? gemm_inst<MODE, 8, true>(a, act, s) : gemm_inst<MODE, 8, false>(a, act, s);
 }
 
-bool int_mfma_rows(Mode mode, int rows, int K) {
+bool int_mfma_rows(const GemmArgs& a) {
   static const int min_rows = [] {
     const char* e = std::getenv("MMF_MFMA_MIN_ROWS");
     return e ? std::atoi(e) : -1;
   }();
-  if (min_rows >= 0) return min_rows > 0 && rows >= min_rows;
-  return rows >= (mode == kFixed ? 3 : 4) || static_cast<int64_t>(rows) * K >= 1024;
+  if (min_rows >= 0) return min_rows > 0 && a.rows >= min_rows;
+  if (a.rows >= 5) return true;
+  const int64_t outs = static_cast<int64_t>(a.p[0].g.N) * (a.epi == kEpiSwigluPair ? 1 : a.nmat);
+  const int K = a.p[0].g.K;
+  const bool fixed = a.mode == kFixed;
+  if (a.rows == 1)
+    return K >= (fixed ? 1024 : 2560) && outs <= (K > 13824 ? 8192 : (!fixed && K >= 4096 ? 49152 : 16384));
+  if (outs >= 49152) return true;
+  if (a.rows == 2 && K < 1024) return fixed && K >= 512 && outs <= 16384;
+  if (fixed && (a.rows == 4 || (a.rows == 3 && K >= 256))) return true;
+  return static_cast<int64_t>(a.rows) * K >= 1024;
 }
 
 hipError_t launch_gemm(const GemmArgs& a, const ActBuf& act, hipStream_t s) {
-  if (a.mode != kFloat && int_mfma_rows(a.mode, a.rows, a.p[0].g.K)) {
+  if (a.mode != kFloat && int_mfma_rows(a)) {
     // (the matrix-core kernel addresses a matrix's planes and weights with 31-bit offsets)
     bool ok = 2 * act.qplane() <= 0x7FFFFFFFu;
     for (int z = 0; z < (a.epi == kEpiSwigluPair ? 1 : a.nmat); ++z)

@@ -18,8 +18,14 @@ SHAPES = [(2, 9, 33), (3, 1025, 70), (5, 4098, 64), (8, 1031, 130), (13, 516, 95
           (520, 1029, 36), (530, 2046, 36), (515, 4099, 36), (514, 6911, 36), (513, 8187, 36), (514, 5632, 36)]
 
 
+# both sides of the integer modes' choice between dot products and matrix cores, one to four rows
+FEW = [(1, 1023, 40), (1, 1025, 40), (1, 1026, 16390), (1, 2559, 40), (1, 2561, 40), (1, 4098, 16390), (1, 13900, 8200),
+       (2, 511, 70), (2, 513, 70), (2, 514, 16390), (2, 1025, 70), (3, 255, 70), (3, 257, 70), (3, 343, 70), (4, 66, 70),
+       (4, 257, 70), (3, 66, 49160)]
+
+
 @pytest.mark.parametrize("mode", [FLOAT, FIXED, INT8])
-@pytest.mark.parametrize("rows,K,N", SHAPES)
+@pytest.mark.parametrize("rows,K,N", SHAPES + FEW)
 def test_bitlinear_odd(eng, oracle, rows, K, N, mode):  # noqa: F811
     print(f"odd rows={rows} K={K} N={N} mode={mode}", flush=True)
     rng = np.random.default_rng(rows + 3 * K + 5 * N + mode)
