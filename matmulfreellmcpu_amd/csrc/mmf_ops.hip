@@ -1320,9 +1320,8 @@ __global__ __launch_bounds__(kBlock) void k_gemm(GemmArgs a, ActBuf act) {
 // come four per chain at a time into one of two register sets, the next four in flight. PAIR: NO
 // = 2, a gate output and its up partner N/2 later (swiglu epilogue).
 // Bound by the chain: K / 8 dependent steps of (R NO + decode) instructions per wave, so R and NO
-// (which share LDS reads and weight decodes) grow only while the launch keeps every SIMD four
-// waves (gemm_f_pick). 16 rows, us per BitLinear call against the 16 x 64 matrix-core tiles: see
-// launch_gemm.
+// (which share LDS reads and weight decodes) grow only while the launch keeps enough waves
+// (gemm_f_form). Against the matrix-core tiles: gemm_f_ok.
 // ------------------------------------------------------------------------------------
 constexpr int kFvWaves = 4;
 
@@ -2228,42 +2227,74 @@ static hipError_t gemm_f_inst(const GemmArgs& a, const ActBuf& act, hipStream_t 
   k_gemm_f<R, NO, PAIR><<<grid, 64 * kFvWaves, static_cast<size_t>(R) * fv_row_floats(act.Lc) * sizeof(float), s>>>(a, act);
   return hipGetLastError();
 }
-// The most outputs per lane that leave four waves per SIMD (a small launch is latency-bound and
-// wants more waves more than fewer LDS reads and decodes); rows of two blocks in a CU's LDS.
-static hipError_t gemm_f_pick(const GemmArgs& a, const ActBuf& act, hipStream_t s) {
+// Rows per block and outputs per lane of a k_gemm_f launch. More of either share LDS reads and weight
+// decodes but leave fewer waves, and rows past the last are computed for nothing; two blocks' rows
+// fit a CU's LDS. Where the lines lie (us per call of each form, over 2656 shapes of 1-2000 rows, K
+// 64-16384, 16-96000 outputs per row): 8 x 2560 x 32000 {1, 1} 49.7, {2, 1} 40.5, {4, 2} 37.4; 6 x 2560 x 32000
+// {2, 2} 32.9, {4, 2} with two of eight rows idle 37.2; 3 x 2560 x 5632 x 3 {1, 1} 18.1, {2, 1} 19.0; two
+// rows a block against one, by the launch's waves at K 512 - 2000: 1536-2560 1.00x, 2560-3072 1.05x,
+// 3072-4096 1.08x; two outputs per lane and one row only for short chains (3 x 64 x 32000 {1, 1} 8.9, {1,
+// 2} 8.1) and rows too long for two (12 x 12000 x 5632 80 -> 77), else level.
+struct FvForm {
+  int R, NO;
+  int64_t waves;  // fewest waves of a launch that takes it
+  int idle;       // ... and at most one idle row per this many
+};
+static FvForm gemm_f_form(const GemmArgs& a, const ActBuf& act) {
+  static constexpr FvForm forms[] = {{4, 2, 3072, 4}, {2, 2, 3072, 4}, {2, 1, 2560, 6}, {1, 2, 4096, 1}};
   const size_t row_lds = static_cast<size_t>(fv_row_floats(act.Lc)) * sizeof(float);
-  auto can = [&](int R, int NO) {
-    return a.rows >= R && gemm_f_waves(a, R, NO) >= 4096 && R * row_lds <= 80 * 1024;
-  };
+  const bool pair = a.epi == kEpiSwigluPair;
+  for (const FvForm& f : forms) {
+    const int pad = (a.rows + f.R - 1) / f.R * f.R - a.rows;
+    const bool fits = f.R == 1 ? act.K < 512 || 2 * row_lds > 80 * 1024 : f.R * row_lds <= 80 * 1024;
+    if (fits && (!pair || f.NO == 2) && f.idle * pad <= a.rows && gemm_f_waves(a, f.R, f.NO) >= f.waves) return f;
+  }
+  return FvForm{1, pair ? 2 : 1, 0, 1};
+}
+
+// Whether a float GEMM runs on the vector ALUs (k_gemm_f), whose time goes with its outputs, rows and
+// columns rounded up to whole blocks, or on the matrix cores, whose time goes with their rounds of
+// tiles: a 16 x 64 tile costs the same for one row as for sixteen, up to 256 of them run at once, and
+// from 384 on 32 x 64 tiles take twice as long per 256. The vector ALUs do about 100000 outputs in
+// the time of one such round; less where LDS holds fewer rows (R = 2, R = 1), over several rounds of
+// short chains (what a launch costs anyway counts once), most where their 32-byte stores lie across
+// two sectors (N % 8 != 0). Measured over the shapes above, matrix
+// cores -> vector ALUs (us per call): 16 x 2048 x 2048 18.3 -> 10.6, 16 x 2560 x 5632 22.3 -> 20.2, 64 x
+// 1024 x 1024 13.3 -> 10.1, 5 x 1024 x 32000 25.4 -> 17.2, 8 x 2560 x 32000 53.5 -> 37.4, 12 x 1024 x 100000
+// 71.7 -> 58.3, 8 x 6912 x 32000 134.7 -> 105.1; past the line 15 x 1024 x 32000 25.4 -> 28.4, 24 x 2560 x 5632
+// 23.5 -> 28.5, 1707 x 2968 x 28 x 3 63.3 -> 79.2, 8 x 6912 x 11264 48.6 -> 50.3, 610 x 15995 x 146 177 -> 242,
+// 12 x 653 x 29403 26.6 -> 29.4, 8 x 71 x 32133 14.5 -> 18.8.
+static bool gemm_f_ok(const GemmArgs& a, const ActBuf& act, const FvForm& f) {
+  const bool pair = a.epi == kEpiSwigluPair;
+  const size_t row_lds = static_cast<size_t>(fv_row_floats(act.Lc)) * sizeof(float);
+  const int64_t nz = pair ? 1 : a.nmat, N = a.p[0].g.N, blocks = (a.rows + f.R - 1) / f.R;
+  if (blocks > 65535 || (pair && N % 16 != 0) || f.R * row_lds > static_cast<size_t>(lds_limit())) return false;
+  // (rows staged for fewer than 64 columns pay as for 64)
+  const int64_t outs = blocks * f.R * (N < 64 ? 64 : (N + 31) / 32 * 32) * nz;
+  const int64_t t16 = (N + 63) / 64 * ((a.rows + 15) / 16) * nz, t32 = (N + 63) / 64 * ((a.rows + 31) / 32) * nz;
+  const double rounds = t16 <= 256 ? 1.0 : (t16 < 384 ? 2.0 : std::max(2.0, t32 / 128.0));
+  const bool across = N % 8 != 0;
+  double line;
+  if (act.K < 512) line = rounds == 1.0 ? 95e3 : (across && act.K < 256 ? 45e3 : 60e3);
+  else if (act.K < 1024 && across && rounds > 1.0) line = 70e3;
+  else line = 4 * row_lds <= 80 * 1024 ? 100e3 : (2 * row_lds <= 80 * 1024 ? 90e3 : 70e3);
+  return static_cast<double>(outs) <= line * rounds;
+}
+
+static hipError_t gemm_f_launch(const GemmArgs& a, const ActBuf& act, const FvForm& f, hipStream_t s) {
   if (a.epi == kEpiSwigluPair) {
-    if (can(4, 2)) return gemm_f_inst<4, 2, true>(a, act, s);
-    if (can(2, 2)) return gemm_f_inst<2, 2, true>(a, act, s);
+    if (f.R == 4) return gemm_f_inst<4, 2, true>(a, act, s);
+    if (f.R == 2) return gemm_f_inst<2, 2, true>(a, act, s);
     return gemm_f_inst<1, 2, true>(a, act, s);
   }
-  if (can(4, 2)) return gemm_f_inst<4, 2, false>(a, act, s);
-  if (can(4, 1)) return gemm_f_inst<4, 1, false>(a, act, s);
-  if (can(2, 2)) return gemm_f_inst<2, 2, false>(a, act, s);
-  if (can(2, 1)) return gemm_f_inst<2, 1, false>(a, act, s);
-  if (can(1, 2)) return gemm_f_inst<1, 2, false>(a, act, s);
-  return gemm_f_inst<1, 1, false>(a, act, s);
-}
-// Float GEMMs of at most kFvOutputs outputs run on the vector ALUs (k_gemm_f): the matrix-core
-// tiles give each SIMD of the chip a chain only from about a hundred 16 x 64 tiles on, and take
-// the same time below. us per BitLinear call, matrix cores (or, up to 15 rows, the FMA kernel
-// before this one) -> vector ALUs: 1 x 1024 x 1024 6.4 -> 5.4, 5 x 2048 x 2048 18.4 -> 8.0, 16 x
-// 2048 x 2048 18.3 -> 10.6, 16 x 5632 x 2048 40.3 -> 21.7, 64 x 1024 x 1024 13.3 -> 10.1, 256 x 300 x
-// 400 11.7 -> 11.5; past it, 96 x 1024 x 1024 13.5 -> 12.0, 24 x 1024 x 5632 13.5 -> 14.6, 48 x
-// 5632 x 2048 43.1 -> 39.6 at 32 rows but 43.9 -> 47.0.
-constexpr int64_t kFvOutputs = 90000;
-
-static bool gemm_f_ok(const GemmArgs& a, const ActBuf& act) {
-  const int64_t outs = static_cast<int64_t>(a.rows) * a.p[0].g.N * (a.epi == kEpiSwigluPair ? 1 : a.nmat);
-  return outs <= kFvOutputs && a.rows <= 65535 && (a.epi != kEpiSwigluPair || a.p[0].g.N % 16 == 0) &&
-         static_cast<size_t>(fv_row_floats(act.Lc)) * sizeof(float) <= static_cast<size_t>(lds_limit());
+  if (f.R == 4) return gemm_f_inst<4, 2, false>(a, act, s);
+  if (f.R == 2) return f.NO == 2 ? gemm_f_inst<2, 2, false>(a, act, s) : gemm_f_inst<2, 1, false>(a, act, s);
+  return f.NO == 2 ? gemm_f_inst<1, 2, false>(a, act, s) : gemm_f_inst<1, 1, false>(a, act, s);
 }
 
 static hipError_t gemm_float(const GemmArgs& a, const ActBuf& act, hipStream_t s) {
-  if (gemm_f_ok(a, act)) return gemm_f_pick(a, act, s);
+  const FvForm f = gemm_f_form(a, act);
+  if (gemm_f_ok(a, act, f)) return gemm_f_launch(a, act, f, s);
   return mfma_f_ok(a) ? launch_gemm_mfma_f(a, act, s) : hipErrorInvalidValue;
 }
 
