@@ -1810,6 +1810,21 @@ __global__ __launch_bounds__(64 * kScWaves) void k_scan_ring(const float* __rest
   if (wave == 0 && sg == 0 && state && live) state[c0 + cl] = s;
 }
 
+// The same for few steps, one thread per column: one load round trip per step (about 0.11 us), where
+// the ring's blocks of 1024 threads and 72 - 100 KB cost 1 us and more a round whatever the steps.
+__global__ __launch_bounds__(256) void k_scan_short(const float* __restrict__ g, const float* __restrict__ in,
+                                                    float* __restrict__ recur, float* __restrict__ state, int T, int H) {
+  const int c = blockIdx.x * 256 + threadIdx.x;
+  if (c >= H) return;
+  float s = state ? state[c] : 0.0f;
+  for (int t = 0; t < T; ++t) {
+    const size_t e = static_cast<size_t>(t) * H + c;
+    s = __builtin_fmaf(g[e], s, in[e]);
+    recur[e] = s;
+  }
+  if (state) state[c] = s;
+}
+
 __global__ void k_copy_ids(const int64_t* __restrict__ src, int64_t* __restrict__ dst, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) dst[i] = src[i];
@@ -2584,9 +2599,20 @@ hipError_t launch_swiglu(const float* a, const float* b, float* out, size_t n, h
   return hipGetLastError();
 }
 
-// (One load round trip per step on D / 256 blocks, the plain loop before the ring scan here, took
-// 136 us at 1000 x 2048; now 12.)
+// Few steps run the plain loop: up to 14 while the ring's blocks of eight columns take the chip in one
+// round with 16-byte transfers (20 with 4-byte ones), 24 (28) in up to two, then one per 18 (9)
+// blocks (us per call, ring -> loop): 1 x 2048 3.4 -> 2.3, 8 x 100 3.8 -> 2.7, 20 x 2560 4.9 -> 4.4, 48 x 4097 9.9
+// -> 8.5, 32 x 8192 8.4 -> 6.1, 64 x 20000 20.9 -> 10.8; past the line 20 x 2048 3.8 -> 4.5, 28 x 4096 5.2 ->
+// 5.5, 64 x 8192 9.8 -> 10.4, 128 x 20000 21.0 -> 33.5, 1000 x 2048 12 -> 136.
 hipError_t launch_scan(const float* i, const float* f, float* out, float* state, int T, int D, hipStream_t s) {
+  const bool wide = D % 8 == 0 && aligned16(f) && aligned16(i);  // scan_ring_launch's 16-byte transfers
+  const int groups = (D + 7) / 8;
+  const int most = groups > 512 ? std::max(wide ? 24 : 28, groups / (wide ? 18 : 9))
+                                : (groups > 256 ? (wide ? 24 : 28) : (wide ? 14 : 20));
+  if (T < kScTT && T <= most) {
+    k_scan_short<<<(D + 255) / 256, 256, 0, s>>>(f, i, out, state, T, D);
+    return hipGetLastError();
+  }
   return scan_ring_launch<false>(f, i, nullptr, out, state, T, D, s);
 }
 

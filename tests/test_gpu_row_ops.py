@@ -88,9 +88,12 @@ def test_swiglu_beyond_a_grid(eng, oracle):  # noqa: F811
         assert_bitexact(got, want, f"swiglu at {e}")
 
 
-# the ring scan (16-byte transfers at D % 8 == 0, aligned; else 4-byte ones) over less than, exactly and more than whole 128-step tiles,
-# and partial column groups
-@pytest.mark.parametrize("T,D,off", [(1, 16, 0), (5, 2048, 0), (127, 64, 0), (128, 64, 0), (129, 48, 0), (1000, 256, 0),
+# the plain loop of few steps and both sides of its lines (by the ring's column groups and transfers,
+# and less than a tile); the ring scan (16-byte transfers at D % 8 == 0, aligned; else 4-byte ones)
+# over less than, exactly and more than whole 128-step tiles, and partial column groups
+@pytest.mark.parametrize("T,D,off", [(14, 256, 0), (15, 256, 0), (20, 257, 0), (21, 257, 0), (20, 64, 1), (21, 64, 1), (24, 2056, 0),
+                                     (25, 2056, 0), (28, 2057, 0), (29, 2057, 0), (57, 4097, 0), (58, 4097, 0), (34, 5000, 0),
+                                     (35, 5000, 0), (127, 20480, 0), (128, 20480, 0), (1, 16, 0), (5, 2048, 0), (127, 64, 0), (128, 64, 0), (129, 48, 0), (1000, 256, 0),
                                      (1, 1, 0), (63, 100, 0), (64, 17, 0), (65, 250, 0), (300, 129, 0), (200, 64, 1), (700, 2056, 0), (700, 2061, 0)])
 def test_scan_sizes(eng, oracle, T, D, off):  # noqa: F811
     print(f"scan T={T} D={D} off={off}", flush=True)
@@ -113,6 +116,10 @@ def test_scan_sizes(eng, oracle, T, D, off):  # noqa: F811
         eng.sync()
         if state is None:
             assert_bitexact(ki.get()[off:].reshape(T, D), want, "scan in place")
+            kx, px = _at(eng, i, off)
+            eng.hgrn_scan(pf, px, pf, T, D, None)  # over the gates
+            eng.sync()
+            assert_bitexact(kf.get()[off:].reshape(T, D), want, "scan in place of the gates")
 
 
 @pytest.mark.parametrize("hidden", [100, 250, 1027])
