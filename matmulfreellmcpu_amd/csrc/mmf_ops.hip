@@ -1877,10 +1877,12 @@ __global__ void k_rownorm(const float* __restrict__ x, const float* __restrict__
 
 // The same with eight consecutive elements per thread and group (t = tid + 256 g: chain position t
 // of every chain), every global input loaded once at entry as 16-byte accesses of any 4-byte
-// alignment, the row kept in registers between the norm chain and the output; t = nb is the tail
-// group. Arithmetic and order are k_rownorm's, which serves rows longer than 8 * 256 * MAXG.
-// Bound by a row's serial phases (load, chain of K / 8 steps, store); 2000 x 2048 10.5 -> 8.1 us
-// (swish gate 14.1 -> 10.6), 1000 x 2056 8.7 -> 6.6, against the element-by-element kernel.
+// alignment, the row kept in registers between the norm chain and the output; the last eight threads
+// take a tail element each (all of them in one thread ran the tail rule's silu up to seven times in a
+// row: swish gate of 1 x 257 4.5 us, now 2.8, 256 x 100 5.4 -> 3.6). Arithmetic and order are
+// k_rownorm's, which serves rows longer than 8 * 256 * MAXG.
+// Bound by a row's serial phases (load, chain of K / 8 steps, store); 2000 x 2048 10.3 -> 7.9 us
+// (swish gate 13.9 -> 10.3), 2000 x 4097 27.4 -> 20.0, against the element-by-element kernel.
 template <int MAXG, bool SW>
 __global__ __launch_bounds__(256) void k_rownorm8(const float* __restrict__ x, const float* __restrict__ o,
                                                   const float* __restrict__ w, float* __restrict__ y, int cols,
@@ -1892,27 +1894,29 @@ __global__ __launch_bounds__(256) void k_rownorm8(const float* __restrict__ x, c
   float* red = X + 8 * LS + 8;
   const size_t r0 = static_cast<size_t>(blockIdx.x) * K;
   auto ld8 = [&](const float* p, int t, float* e) {
-    if (t < nb) {
-      const f4u l = reinterpret_cast<const f4u*>(p + 8 * t)[0], h = reinterpret_cast<const f4u*>(p + 8 * t)[1];
+    const f4u l = reinterpret_cast<const f4u*>(p + 8 * t)[0], h = reinterpret_cast<const f4u*>(p + 8 * t)[1];
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        e[c] = l[c];
-        e[4 + c] = h[c];
-      }
-    } else {
-#pragma unroll
-      for (int c = 0; c < 8; ++c) e[c] = p[K8 + (c < nt ? c : 0)];
+    for (int c = 0; c < 4; ++c) {
+      e[c] = l[c];
+      e[4 + c] = h[c];
     }
   };
-  const int G = nb + (nt > 0 ? 1 : 0);
+  const int te = tid - 248;  // this thread's tail element
+  const bool tail = te >= 0 && te < nt;
   float xv[MAXG][8], wv[MAXG][8], ov[SW ? MAXG : 1][8];
 #pragma unroll
   for (int g = 0; g < MAXG; ++g) {
     const int t = tid + 256 * g;
-    if (t >= G) continue;
+    if (t >= nb) continue;
     ld8(x + r0, t, xv[g]);
     ld8(w, t, wv[g]);
     if constexpr (SW) ld8(o + r0, t, ov[g]);
+  }
+  float xt = 0.0f, wt = 0.0f, ot = 0.0f;
+  if (tail) {
+    xt = x[r0 + K8 + te];
+    wt = w[K8 + te];
+    if constexpr (SW) ot = o[r0 + K8 + te];
   }
   for (int j = 0; j < 8; ++j)
     for (int t = nb + tid; t < L32; t += 256) X[j * LS + t] = 0.0f;
@@ -1920,13 +1924,11 @@ __global__ __launch_bounds__(256) void k_rownorm8(const float* __restrict__ x, c
 #pragma unroll
   for (int g = 0; g < MAXG; ++g) {
     const int t = tid + 256 * g;
-    if (t >= G) continue;
+    if (t >= nb) continue;
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      if (t < nb) X[c * LS + t] = xv[g][c];
-      else if (c < nt) X[8 * LS + c] = xv[g][c];
-    }
+    for (int c = 0; c < 8; ++c) X[c * LS + t] = xv[g][c];
   }
+  if (tail) X[8 * LS + te] = xt;
   __syncthreads();
   if (tid < 64) __builtin_amdgcn_s_setprio(3);
   const float r = rstd_of(block_sumsq_ring(X, Lc, LS, nt, red), K, eps);
@@ -1934,22 +1936,21 @@ __global__ __launch_bounds__(256) void k_rownorm8(const float* __restrict__ x, c
 #pragma unroll
   for (int g = 0; g < MAXG; ++g) {
     const int t = tid + 256 * g;
-    if (t >= G) continue;
+    if (t >= nb) continue;
     float v[8];
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
       v[c] = (xv[g][c] * r) * wv[g][c];
-      if (SW) v[c] = v[c] * silu_of(ov[SW ? g : 0][c], t >= nb);
+      if (SW) v[c] = v[c] * silu_of(ov[SW ? g : 0][c], false);
     }
     float* yo = y + r0 + 8 * t;
-    if (t < nb) {
-      reinterpret_cast<f4u*>(yo)[0] = f4u{v[0], v[1], v[2], v[3]};
-      reinterpret_cast<f4u*>(yo)[1] = f4u{v[4], v[5], v[6], v[7]};
-    } else {
-#pragma unroll
-      for (int c = 0; c < 7; ++c)
-        if (c < nt) yo[c] = v[c];
-    }
+    reinterpret_cast<f4u*>(yo)[0] = f4u{v[0], v[1], v[2], v[3]};
+    reinterpret_cast<f4u*>(yo)[1] = f4u{v[4], v[5], v[6], v[7]};
+  }
+  if (tail) {
+    float v = (xt * r) * wt;
+    if (SW) v = v * silu_of(ot, true);
+    y[r0 + K8 + te] = v;
   }
 }
 
@@ -2558,12 +2559,12 @@ hipError_t launch_embed(const float* emb, const int64_t* ids, float* h, int rows
 template <bool SW>
 static hipError_t rownorm_launch(const float* x, const float* o, const float* w, float* y, int rows, int cols,
                                  float eps, hipStream_t s) {
-  const int nb = (cols & ~7) / 8, Lc = nb > 0 ? (nb + 15) / 16 * 16 : 16, G = nb + (cols % 8 ? 1 : 0);
+  const int nb = (cols & ~7) / 8, Lc = nb > 0 ? (nb + 15) / 16 * 16 : 16;
   // (the ring chains read up to 32 floats past the tail)
   const size_t lds = (static_cast<size_t>(8 * host_lds_stride(Lc) + 8) + 32) * sizeof(float);
-  if (G <= 256) k_rownorm8<1, SW><<<rows, 256, lds, s>>>(x, o, w, y, cols, eps);
-  else if (G <= 512) k_rownorm8<2, SW><<<rows, 256, lds, s>>>(x, o, w, y, cols, eps);
-  else if (G <= 1024) k_rownorm8<4, SW><<<rows, 256, lds, s>>>(x, o, w, y, cols, eps);
+  if (nb <= 256) k_rownorm8<1, SW><<<rows, 256, lds, s>>>(x, o, w, y, cols, eps);
+  else if (nb <= 512) k_rownorm8<2, SW><<<rows, 256, lds, s>>>(x, o, w, y, cols, eps);
+  else if (nb <= 1024) k_rownorm8<4, SW><<<rows, 256, lds, s>>>(x, o, w, y, cols, eps);
   else k_rownorm<<<rows, 256, lds, s>>>(x, SW ? o : nullptr, w, y, cols, eps);
   return hipGetLastError();
 }
