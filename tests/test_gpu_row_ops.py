@@ -53,7 +53,7 @@ def test_swishgate_without_gate(eng, oracle, cols):  # noqa: F811
     assert_bitexact(y.get(), oracle.rmsnorm(x, w, 1e-6), "norm")
 
 
-@pytest.mark.parametrize("n", [1, 7, 8, 12, 1023, 1024, 1029, 100003])
+@pytest.mark.parametrize("n", [1, 7, 8, 12, 1016, 1020, 1023, 1024, 1029, 100003])
 def test_swiglu_sizes(eng, oracle, n):  # noqa: F811
     rng = np.random.default_rng(n)
     a, b = (rng.standard_normal(n).astype(np.float32) * 4 for _ in range(2))
