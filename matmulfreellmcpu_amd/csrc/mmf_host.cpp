@@ -801,6 +801,15 @@ void decode_step(mmf_ctx* c, Model& m) {
   }
 }
 
+// Whether a fused serving step's lm_head runs on the decode kernel, where every block recomputes its
+// stream's final norms, or on the row prologue and GEMM. Steps of four layers (us, decode kernel /
+// row lm_head): 2 streams of the 370M width, vocabulary 32000, float 114 / 112, FixedQ510 117 / 117, of the
+// 1.3B width 187 / 187 and 185 / 189; 4 of the 370M width float 134 / 138, FixedQ510 144 / 135, Int8Absmax 147 / 133, at
+// vocabulary 8000 118 / 119, 128 / 126 and 129 / 128; 5 of width 512 float 126 / 123, 8 of the 370M width 180 / 165.
+bool lm_fused(const Model& m, size_t B) {
+  return B <= 2 || (B <= 4 && (m.mode == kFloat || m.cfg.vocab_size <= 8192));
+}
+
 // The fused serving step's vectors for B streams, zeroed where they grew (their padding stays
 // zero: only valid positions are ever written).
 void alloc_step(mmf_ctx* c, Model& m, size_t B) {
@@ -812,28 +821,26 @@ void alloc_step(mmf_ctx* c, Model& m, size_t B) {
     b->get(n);
     MMF_HIP(hipMemsetAsync(b->p, 0, n, c->stream));
   }
-  s.keys.as<unsigned long long>(B * kLMBlocks);
+  if (lm_fused(m, B)) s.keys.as<unsigned long long>(B * kLMBlocks);
 }
-
-// Most streams whose lm_head runs on the decode kernel, where every block recomputes its stream's
-// final norms; more take the row prologue and GEMM. Measured steps (four layers, vocabulary
-// 32000, float / FixedQ510): 4 streams of the 2.7B width 383 / 396 us against 431 / 425 with the
-// row lm_head; 8 streams of the 370M width 196 / 210 against 175 / 186.
-constexpr size_t kLMFusedMax = 4;
 
 // Whether the serving step of B streams runs on the fused decode kernels: half the row path's
 // launches, but every block recomputes its stream's norms, so their time grows with B times the
-// width while the row path's hardly grows. Steps of four layers, row path -> fused (us):
-//   integer modes: 1 stream of the 1.3B width FixedQ510 319 -> 161, 8 x 370M 201 -> 188, 10 x 370M
-//   205 -> 204, 3 x 1.3B 266 -> 261, 4 x 1.3B 268 -> 288, 2 x 2.7B 290 -> 278, 3 x 2.7B 296 -> 307;
-//   float: 1 x 370M 159 -> 121, 12 x 370M 220 -> 206, 3 x 1.3B 286 -> 243, 4 x 1.3B 287 -> 303,
-//   2 x 2.7B 274 -> 279, 24 x 370M 246 -> 294.
+// width while the row path's hardly grows. Steps of four layers, vocabulary 32000, row path -> fused (us):
+//   integer modes: 128 streams of width 64 FixedQ510 197 -> 168, Int8Absmax 210 -> 185; 32 of width 256 196 ->
+//   162 and 200 -> 179; 16 of width 512 188 -> 174 and 198 -> 189; 8 x 370M 184 -> 172 and 176 -> 168, 10 x 370M 190
+//   -> 190 and 180 -> 187; 4 of width 1536 249 -> 219 and 249 -> 225; 3 x 1.3B 250 -> 245 and 228 -> 236; 2 x
+//   2.7B 273 -> 258 and 250 -> 269;
+//   float: 128 of width 64 180 -> 141, 32 of width 256 159 -> 125, 12 x 370M 206 -> 188, 16 x 370M 216 -> 222,
+//   3 x 1.3B 268 -> 228, 2 x 2.7B 260 -> 260.
 // Several streams need H % 8 == 0, so that no element of the gate math over all B * H elements
 // is a SIMD tail element (the row path's rule). The kernels must fit the widths.
 bool step_fused(const Model& m, size_t B) {
   const size_t H = m.cfg.hidden_size;
   const Mode mode = static_cast<Mode>(m.mode);
-  const size_t most = H > 1024 ? 6144 : (mode == kFloat ? 12288 : 9216);
+  size_t most;
+  if (H <= 1024) most = mode == kFloat ? 12288 : 9216;
+  else most = H > 1536 && (mode == kInt8 || (mode == kFloat && H > 2048)) ? 4096 : 6144;
   if (m.ext_on() || (B > 1 && (H % 8 != 0 || B * H > most))) return false;
   for (DecKind k : {kIFG, kO, kGate, kLM})
     if (!decode_fits(k, mode, m.gH)) return false;
@@ -1800,13 +1807,14 @@ namespace {
 // The launches of one lockstep serving step of the m.streams streams: embedding of the
 // device tokens d, every layer over the B rows, final norm + lm_head into lg, argmax into am.
 // Few streams (step_fused) run the fused decode kernels, four launches per layer over a grid of
-// (blocks, streams); the lm_head of one stream is the decode kernel's, of several the row one.
+// (blocks, streams), the lm_head by lm_fused.
 void step_kernels(mmf_ctx* c, Model& m, const int64_t* d, float* h, float* lg, int64_t* am) {
   const size_t B = m.streams, H = m.cfg.hidden_size, V = m.cfg.vocab_size;
   if (step_fused(m, B)) {
+    const bool lm = lm_fused(m, B);
     for (size_t l = 0; l < m.layers.size(); ++l)
-      for (DecKind k : {kIFG, kO, kGate, kDown}) decode_one(c, m, k, l, true, B, d, B > kLMFusedMax ? h : nullptr);
-    if (B <= kLMFusedMax) {
+      for (DecKind k : {kIFG, kO, kGate, kDown}) decode_one(c, m, k, l, true, B, d, lm ? nullptr : h);
+    if (lm) {
       DecArgs a = dec_base(m);
       set_proj(c, m, a, 0, m.lm);
       a.x = static_cast<const float*>(m.ss.h.p);

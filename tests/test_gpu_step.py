@@ -10,11 +10,12 @@ pytestmark = pytest.mark.gpu
 FLOAT, FIXED, INT8 = 0, 1, 2
 
 # (blob, streams): one stream (with SIMD tails on "odd"), the lm_head's switch to the row kernels
-# (4 / 5), and the last fused and first row step of each width and mode
+# (4 / 5; 2 / 3 for the integer modes beyond vocabulary 8192), and the last fused and first row step
+# of each width and mode
 CASES = [("odd", 1, FLOAT), ("odd", 1, FIXED), ("odd", 1, INT8), ("odd", 2, FLOAT),
          ("small", 1, FLOAT), ("small", 4, FIXED), ("small", 5, INT8), ("small", 49, FLOAT), ("small", 37, FIXED),
          ("wide", 12, FLOAT), ("wide", 13, FLOAT), ("wide", 9, FIXED), ("wide", 10, INT8),
-         ("h2048", 1, FIXED), ("h2048", 3, INT8), ("h2048", 4, FIXED), ("h2048", 3, FLOAT), ("h2048", 4, FLOAT),
+         ("h2048", 1, FIXED), ("h2048", 2, INT8), ("h2048", 3, INT8), ("h2048", 3, FIXED), ("h2048", 4, FIXED), ("h2048", 3, FLOAT), ("h2048", 4, FLOAT),
          ("h2560", 2, FIXED), ("h2560", 3, INT8), ("h2560", 2, FLOAT), ("h2560", 1, INT8)]
 
 
