@@ -1328,6 +1328,7 @@ hipError_t launch_argmax_keys(const unsigned long long* keys, int n, int streams
 }
 
 hipError_t launch_decode(DecKind kind, Mode mode, const DecArgs& a, hipStream_t s) {
+  if (kind == kIFG && is_step(a) && !a.x && !a.tokens) return hipErrorInvalidValue;
   switch (mode) {
     case kFloat: return dec_mode<kFloat>(kind, a, s);
     case kFixed: return dec_mode<kFixed>(kind, a, s);

@@ -92,11 +92,11 @@ struct DecArgs {
                           // are copied into LDS at entry (0: read from global in the GEMV)
   int32_t* acc;           // kOp, integer modes: the int32 accumulators [N] (tails and the
                           // Q5.10 bias included), or null
-  // A serving step of `streams` independent streams (0 or 1: one): blockIdx.y is the stream.
-  // Every vector above is then an array of streams, 8*Lc + 8 floats apart (state: H apart,
-  // logits: vocab apart, keys: kLMBlocks apart).
+  // 0: the batch-1 decode, whose layer-0 token is the largest of *keys. Else a serving step of this
+  // many independent streams: blockIdx.y is the stream, and every vector above is an array of
+  // streams, 8*Lc + 8 floats apart (state: H apart, logits: vocab apart, keys: kLMBlocks apart).
   int streams;
-  const int64_t* tokens;  // kIFG layer 0: the streams' tokens (in [0, vocab)), or null: *key
+  const int64_t* tokens;  // the streams' tokens (in [0, vocab)): a serving step's kIFG reads them where x is null
   int out_nat;            // kDown: out is [streams][N] in natural order (the row lm_head's input)
 };
 
@@ -111,6 +111,7 @@ inline int lm_blocks(int groups, int K) {
   const int cap = K <= 1024 ? kLMBlocks : 512;
   return groups < cap ? groups : cap;
 }
+// (hipErrorInvalidValue: a serving step's kIFG with neither x nor tokens)
 hipError_t launch_decode(DecKind kind, Mode mode, const DecArgs& a, hipStream_t s);
 // Whether launch_decode has a launch for this kind over geometry g (rows that fit the block
 // layout and LDS).
