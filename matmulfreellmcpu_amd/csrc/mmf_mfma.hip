@@ -934,12 +934,21 @@ struct Plan {
   int fm = 2;  // 32-row fragments per wave (1: 32-row tiles)
 };
 constexpr int kGroupStages = 216, kFewStages = 144;
+// MMF_KW8_32=0: GEMMs of 8-32 rows split K instead of taking the eight-K-group tiles (comparisons).
+static bool kw8_rows32() {
+  static const bool on = [] {
+    const char* e = std::getenv("MMF_KW8_32");
+    return !(e && e[0] == '0');
+  }();
+  return on;
+}
 
 Plan plan_of(const GemmArgs& a) {
   const int nz = (a.epi == kEpiSwigluPair) ? 1 : a.nmat;
   const int nst = a.p[0].g.Lc / 8;
   const int t32 = tiles_of<1, 1, 1>(a) * nz, t64 = tiles_of<1, 1>(a) * nz;
-  const bool split = nst > kGroupStages || (nst > kFewStages && a.rows <= 40 && tiles_of<1, 2>(a) * nz <= 8);
+  const bool split = nst > kGroupStages || (nst > kFewStages && a.rows <= 40 && tiles_of<1, 2>(a) * nz <= 8) ||
+                     (!kw8_rows32() && a.rows >= 8 && a.rows <= 32);
   if (!split) {
     const bool two = a.p[0].g.K >= 512;  // a second round of tiles
     if (t32 <= 256) return Plan{1, 1, 1, 8, 1};

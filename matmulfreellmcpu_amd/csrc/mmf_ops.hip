@@ -1321,7 +1321,7 @@ __global__ __launch_bounds__(kBlock) void k_gemm(GemmArgs a, ActBuf act) {
 // = 2, a gate output and its up partner N/2 later (swiglu epilogue).
 // Bound by the chain: K / 8 dependent steps of (R NO + decode) instructions per wave, so R and NO
 // (which share LDS reads and weight decodes) grow only while the launch keeps enough waves
-// (gemm_f_form). Against the matrix-core tiles: gemm_f_ok.
+// (gemm_f_form). Against the matrix-core tiles: gemm_f_line.
 // ------------------------------------------------------------------------------------
 constexpr int kFvWaves = 4;
 
@@ -2287,11 +2287,10 @@ static FvForm gemm_f_form(const GemmArgs& a, const ActBuf& act) {
 // 71.7 -> 58.3, 8 x 6912 x 32000 134.7 -> 105.1; past the line 15 x 1024 x 32000 25.4 -> 28.4, 24 x 2560 x 5632
 // 23.5 -> 28.5, 1707 x 2968 x 28 x 3 63.3 -> 79.2, 8 x 6912 x 11264 48.6 -> 50.3, 610 x 15995 x 146 177 -> 242,
 // 12 x 653 x 29403 26.6 -> 29.4, 8 x 71 x 32133 14.5 -> 18.8.
-static bool gemm_f_ok(const GemmArgs& a, const ActBuf& act, const FvForm& f) {
+static bool gemm_f_line(const GemmArgs& a, const ActBuf& act, const FvForm& f) {
   const bool pair = a.epi == kEpiSwigluPair;
   const size_t row_lds = static_cast<size_t>(fv_row_floats(act.Lc)) * sizeof(float);
   const int64_t nz = pair ? 1 : a.nmat, N = a.p[0].g.N, blocks = (a.rows + f.R - 1) / f.R;
-  if (blocks > 65535 || (pair && N % 16 != 0) || f.R * row_lds > static_cast<size_t>(lds_limit())) return false;
   // (rows staged for fewer than 64 columns pay as for 64)
   const int64_t outs = blocks * f.R * (N < 64 ? 64 : (N + 31) / 32 * 32) * nz;
   const int64_t t16 = (N + 63) / 64 * ((a.rows + 15) / 16) * nz, t32 = (N + 63) / 64 * ((a.rows + 31) / 32) * nz;
@@ -2302,6 +2301,11 @@ static bool gemm_f_ok(const GemmArgs& a, const ActBuf& act, const FvForm& f) {
   else if (act.K < 1024 && across && rounds > 1.0) line = 70e3;
   else line = 4 * row_lds <= 80 * 1024 ? 100e3 : (2 * row_lds <= 80 * 1024 ? 90e3 : 70e3);
   return static_cast<double>(outs) <= line * rounds;
+}
+
+static bool gemm_f_fits(const GemmArgs& a, const ActBuf& act, const FvForm& f) {
+  return (a.rows + f.R - 1) / f.R <= 65535 && (a.epi != kEpiSwigluPair || a.p[0].g.N % 16 == 0) &&
+         f.R * static_cast<size_t>(fv_row_floats(act.Lc)) * sizeof(float) <= static_cast<size_t>(lds_limit());
 }
 
 static hipError_t gemm_f_launch(const GemmArgs& a, const ActBuf& act, const FvForm& f, hipStream_t s) {
@@ -2315,9 +2319,15 @@ static hipError_t gemm_f_launch(const GemmArgs& a, const ActBuf& act, const FvFo
   return f.NO == 2 ? gemm_f_inst<1, 2, false>(a, act, s) : gemm_f_inst<1, 1, false>(a, act, s);
 }
 
+// MMF_FLOAT_MFMA_MIN_ROWS: the matrix cores from this many rows on (0: never) instead of by gemm_f_line.
 static hipError_t gemm_float(const GemmArgs& a, const ActBuf& act, hipStream_t s) {
+  static const int min_rows = [] {
+    const char* e = std::getenv("MMF_FLOAT_MFMA_MIN_ROWS");
+    return e ? std::atoi(e) : -1;
+  }();
   const FvForm f = gemm_f_form(a, act);
-  if (gemm_f_ok(a, act, f)) return gemm_f_launch(a, act, f, s);
+  const bool vec = min_rows >= 0 ? min_rows == 0 || a.rows < min_rows : gemm_f_line(a, act, f);
+  if (vec && gemm_f_fits(a, act, f)) return gemm_f_launch(a, act, f, s);
   return mfma_f_ok(a) ? launch_gemm_mfma_f(a, act, s) : hipErrorInvalidValue;
 }
 

@@ -1,6 +1,10 @@
 """BitLinear at widths and row addresses that fit no vector load or tile, against the CPU
 restatement, bit for bit: the float4-free row prologue, the tail terms and the partial tiles of
 the integer matrix-core epilogues."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -119,3 +123,42 @@ def test_serve_odd_hidden(tmp_path, oracle, hidden, mode):
         np.testing.assert_array_equal(np.array(g), w)
     assert_bitexact(e.state(), wst, "states")
     e.close()
+
+
+CHILD = """
+import hashlib, sys
+import numpy as np
+sys.path[:0] = [{root!r}, {tests!r}]
+from matmulfreellmcpu_amd import Engine
+from test_gpu_parity import Dev
+rng, e, h = np.random.default_rng(9), Engine(0), hashlib.md5()
+for rows, K, N in ((20, 2048, 512), (3, 530, 70), (40, 1000, 3000)):
+    x = rng.standard_normal((rows, K)).astype(np.float32)
+    pid = e.register_proj(rng.integers(-1, 2, (N, K)).astype(np.int8), 30.0, np.ones(K, np.float32))
+    dx, dout = Dev(e, x), Dev(e, shape=(rows, N))
+    for mode in (0, 1, 2):
+        e.bitlinear(pid, dx.ptr, dout.ptr, rows, mode=mode)
+        e.sync()
+        h.update(dout.get().tobytes())
+print("RESULT", h.hexdigest(), e.workspace_bytes())
+"""
+
+
+def test_switches():
+    """MMF_KW8_32=0 splits K at 8-32 rows (the partials are workspace), MMF_FLOAT_MFMA_MIN_ROWS moves
+    the float line; the results stay the same bits."""
+    here = os.path.dirname(os.path.abspath(__file__))
+    code = CHILD.format(root=os.path.dirname(here), tests=here)
+
+    def run(**env):
+        print(f"switches {env}", flush=True)
+        r = subprocess.run([sys.executable, "-c", code], env={**os.environ, **env}, capture_output=True, text=True, timeout=100)
+        assert r.returncode == 0, r.stderr[-2000:]
+        line = [ln for ln in r.stdout.splitlines() if ln.startswith("RESULT")][0].split()
+        return line[1], int(line[2])
+
+    plain, ws = run()
+    split, ws_split = run(MMF_KW8_32="0")
+    assert split == plain and ws_split > ws
+    for n in ("0", "1", "30"):
+        assert run(MMF_FLOAT_MFMA_MIN_ROWS=n) == (plain, ws)
