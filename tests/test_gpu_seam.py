@@ -3,7 +3,7 @@ three to a launch, codes of every 16-bit value, widths off every vector size, ro
 import numpy as np
 import pytest
 
-from test_gpu_parity import eng  # noqa: F401  (module fixture)
+from test_gpu_parity import Dev, eng  # noqa: F401  (module fixture)
 
 pytestmark = pytest.mark.gpu
 
@@ -27,5 +27,25 @@ def test_seam_shapes(eng, case):  # noqa: F811
             want = (x.astype(np.float64) @ w.T.astype(np.float64)).astype(np.int64)  # |sums| < 2^53: exact
             np.testing.assert_array_equal(g, want.astype(np.int32))
         xs = [x[::-1].copy() for x in xs]
+    for p in pids:
+        eng.proj_release(p)
+
+
+def test_long_rows(eng):  # noqa: F811
+    """Rows whose planes do not fit LDS, two projections of one shape (the second's planes and tail
+    codes follow the first's), through the host seam and on device buffers."""
+    b, K, N = 5, 82005, 20
+    print(f"seam long rows {b} x {K} x {N}", flush=True)
+    rng = np.random.default_rng(K)
+    ws = [rng.integers(-1, 2, (N, K)).astype(np.int8) for _ in range(2)]
+    xs = [rng.integers(-2000, 2001, (b, K)).astype(np.int32) for _ in range(2)]
+    want = [(x.astype(np.float64) @ w.T.astype(np.float64)).astype(np.int32) for x, w in zip(xs, ws)]  # exact below 2^53
+    pids = [eng.register_proj(w, 10.0) for w in ws]
+    for got, wz in zip(eng.ternary_matmul_host(pids, xs), want):
+        np.testing.assert_array_equal(got, wz)
+    dx, dacc = Dev(eng, xs[1]), Dev(eng, shape=(b, N), dtype=np.int32)
+    eng.ternary_matmul(pids[1], dx.ptr, dacc.ptr, b)
+    eng.sync()
+    np.testing.assert_array_equal(dacc.get(), want[1])
     for p in pids:
         eng.proj_release(p)

@@ -81,10 +81,11 @@ def _case(eng, oracle, rows, K, N, mode, seed):
         np.testing.assert_array_equal(outs["noalloc"][1], want["acc"])
 
 
-# (rows, K, N): the first call of each pair is the larger one. 300 rows take the matrix
-# cores; 40 rows x K 2048 split K over 8 blocks in the integer modes (partials in the
-# scratch); 1 row is the single-row path; K 1031 leaves a 7-element tail.
-PAIRS = [((300, 2816, 1024), (40, 2048, 512)), ((40, 2048, 512), (1, 1031, 96)), ((130, 1024, 333), (17, 256, 128))]
+# (rows, K, N): the first call of each pair is the larger one. 300 and 40 rows take the matrix
+# cores; 100 rows x K 14003 and 20 x 9990 split K in the integer modes (partials in the scratch);
+# 1 row is the single-row path; K 1031 leaves a 7-element tail.
+PAIRS = [((300, 2816, 1024), (40, 2048, 512)), ((40, 2048, 512), (1, 1031, 96)), ((130, 1024, 333), (17, 256, 128)),
+         ((100, 14003, 300), (20, 9990, 130)), ((20, 9990, 130), (40, 2048, 512))]
 
 
 @pytest.mark.parametrize("first,second", PAIRS)
@@ -103,7 +104,7 @@ def test_noalloc_allocates_nothing(oracle, mode):
     from matmulfreellmcpu_amd import Engine
     e = Engine(0)
     try:
-        rows, K, N = 40, 2048, 512  # the integer modes split K here: partials in the scratch too
+        rows, K, N = 20, 9990, 130  # the integer modes split K here: partials in the scratch too
         rng = np.random.default_rng(31 + mode)
         x = rng.standard_normal((rows, K)).astype(np.float32)
         nw = np.ones(K, np.float32)
@@ -118,7 +119,8 @@ def test_noalloc_allocates_nothing(oracle, mode):
         assert_bitexact(dout.get(), oracle.bitlinear(x, nw, wq, 25.0, 1e-6, mode)["out"], "noalloc on a fresh context")
         e.bitlinear(pid, dx.ptr, dout.ptr, rows, mode=mode)
         e.sync()
-        assert e.workspace_bytes() > 0
+        # the activations (codes of 32 rows), and 16 splits of partials
+        assert e.workspace_bytes() >= (rows * K * 4 if mode == FLOAT else 32 * K + 16 * rows * N * 4)
         dx.free()
         dout.free()
     finally:
