@@ -256,13 +256,15 @@ size_t gemm_workspace_bytes(const GemmArgs& a);
 // where K is long against the tile's fixed cost, and one row only while its 32 x 64 tiles fit one
 // round (us per call, dot products -> matrix cores; 5 rows and more: always).
 //   1 row: FixedQ510 from K 1024, Int8Absmax from 2560, up to 16384 outputs (Int8Absmax from K 4096
-//     on 49152; 8192 beyond K 13824, where the tiles split K): 4096 x 5632 FixedQ510 17.4 -> 13.0,
-//     9000 x 32000 Int8Absmax 36.4 -> 27.4; but 1024 x 16896 FixedQ510 9.3 -> 13.7, 7396 x 60675 64 ->
-//     78, 2048 x 7116 Int8Absmax 9.6 -> 9.8.
-//   2 - 4 rows: rows * K >= 1024 (FixedQ510: 3 rows from K 256, 4 rows always, 2 rows below K 1024 to
-//     16384 outputs only; Int8Absmax: 2 rows from K 1024): 2 x 1024 x 5632 FixedQ510 12.4 -> 8.1; but 2 x 512 x
-//     16896 11.4 -> 12.4, 3 x 64 x 20225 8.5 -> 9.1, 4 x 64 x 256 Int8Absmax 8.1 -> 8.3. Or 49152
-//     outputs: 3 x 64 x 100000 FixedQ510 14.0 -> 9.8; but 2 x 64 x 33792 9.3 -> 9.8.
+//     on, or with tail elements, 49152; 8192 beyond 216 stages, where the tiles split K): 4096 x 5632
+//     FixedQ510 17.4 -> 13.0, 9000 x 32000 Int8Absmax 36.4 -> 27.4; but 1024 x 16896 FixedQ510 9.3 -> 13.7, 7396 x
+//     60675 64 -> 78, 2048 x 7116 Int8Absmax 9.6 -> 9.8.
+//   2 rows from K 560 (512 with tail elements, or FixedQ510 to 16384 outputs): 2 x 1024 x 5632 FixedQ510
+//     12.4 -> 8.1, 2 x 632 x 45870 17.8 -> 14.8; but 2 x 512 x 16896 11.4 -> 12.4.
+//   3 and 4 rows: K 342 and 256; with tail elements, which the dot products take one by one, FixedQ510
+//     always and Int8Absmax 4 rows; FixedQ510 4 rows always and 3 beyond K 128: 3 x 145 x 636 x 3 10.8 -> 10.1,
+//     3 x 152 x 9776 9.1 -> 8.1; but 3 x 64 x 20225 8.5 -> 9.1, 4 x 64 x 256 Int8Absmax 8.1 -> 8.3.
+//   2 - 4 rows of 49152 outputs: 3 x 64 x 100000 FixedQ510 14.0 -> 9.8; but 2 x 64 x 33792 9.3 -> 9.8.
 // MMF_MFMA_MIN_ROWS sets another row count (0: never).
 bool int_mfma_rows(const GemmArgs& a);
 // HGRN gate + recurrence over rows (hgrn_model.cpp:109-150). i, f, g: [rows, H].

@@ -923,11 +923,12 @@ bool mfma_launch(const GemmArgs& a, const ActBuf& act, dim3 grid, hipStream_t s)
 // columns when that still gives every CU a block (all blocks of all matrices), else 128.
 // K is split in powers of two until there are 128 blocks (each split >= 4 stages) where the eight
 // waves of one block would walk too many stages: beyond kGroupStages stages of 64 elements (K
-// 13824), and beyond kFewStages (K 9216) for at most 40 rows of at most eight 64 x 128 tiles, whose
-// 16 splits have 32 waves where a K-group tile has eight (us per call, K-groups -> split: 8 x 12288
-// x 256 FixedQ510 24.2 -> 23.1, Int8Absmax 22.8 -> 21.2, 8 x 13824 x 1024 27.0 -> 25.0 and 25.1 ->
-// 22.6; but 32 x 8836 x 1024 21.7 -> 22.8 and 20.3 -> 21.1, at 64 rows 12288 x 1024 25.0 -> 26.7 and
-// 23.4 -> 24.0, at 16 tiles, 8 x 13824 x 2048, 27.0 -> 29.1 and 25.3 -> 25.1). Between the two limits
+// 13824), and beyond kFewStages (K 9216) for at most 40 rows of one matrix of at most eight 64 x 128
+// tiles (16 rows: 14), whose splits have four times a K-group tile's waves (us per call, K-groups ->
+// split: 8 x 12288 x 256 FixedQ510 24.2 -> 23.1, Int8Absmax 22.8 -> 21.2, 8 x 13824 x 1024 27.0 -> 25.0 and
+// 25.1 -> 22.6, 8 x 13824 x 1792 26.9 -> 25.1 and 25.2 -> 23.4; but 32 x 8836 x 1024 21.7 -> 22.8 and 20.3 ->
+// 21.1, 40 x 13824 x 1792 27.6 -> 28.7, at 64 rows 12288 x 1024 25.0 -> 26.7 and 23.4 -> 24.0, at 16 tiles, 8
+// x 13824 x 2048, 27.0 -> 29.1 and 25.3 -> 25.1, three matrices 21 x 9617 x 60 24.5 -> 25.9). Between the two limits
 // everything else keeps the K-groups: 100 x 13824 x 4096 32.6 -> 48.9, 16 x 12288 x 4096 25.1 -> 37.8.
 struct Plan {
   int wm, wn, ksplit, kw;
@@ -947,7 +948,8 @@ Plan plan_of(const GemmArgs& a) {
   const int nz = (a.epi == kEpiSwigluPair) ? 1 : a.nmat;
   const int nst = a.p[0].g.Lc / 8;
   const int t32 = tiles_of<1, 1, 1>(a) * nz, t64 = tiles_of<1, 1>(a) * nz;
-  const bool split = nst > kGroupStages || (nst > kFewStages && a.rows <= 40 && tiles_of<1, 2>(a) * nz <= 8) ||
+  const bool few = a.rows <= 40 && nz == 1 && tiles_of<1, 2>(a) <= (a.rows <= 16 ? 14 : 8);
+  const bool split = nst > kGroupStages || (nst > kFewStages && few) ||
                      (!kw8_rows32() && a.rows >= 8 && a.rows <= 32);
   if (!split) {
     const bool two = a.p[0].g.K >= 512;  // a second round of tiles

@@ -2349,11 +2349,13 @@ bool int_mfma_rows(const GemmArgs& a) {
   const int64_t outs = static_cast<int64_t>(a.p[0].g.N) * (a.epi == kEpiSwigluPair ? 1 : a.nmat);
   const int K = a.p[0].g.K;
   const bool fixed = a.mode == kFixed;
+  const bool tail = K % 8 != 0;  // (the dot products take the tail elements one by one)
   if (a.rows == 1)
-    return K >= (fixed ? 1024 : 2560) && outs <= (K > 13824 ? 8192 : (!fixed && K >= 4096 ? 49152 : 16384));
+    return K >= (fixed ? 1024 : 2560) &&
+           outs <= (a.p[0].g.Lc > 1728 ? 8192 : (!fixed && (tail || K >= 4096) ? 49152 : 16384));
   if (outs >= 49152) return true;
-  if (a.rows == 2 && K < 1024) return fixed && K >= 512 && outs <= 16384;
-  if (fixed && (a.rows == 4 || (a.rows == 3 && K >= 256))) return true;
+  if (a.rows == 2) return K >= 560 || (K >= 512 && (tail || (fixed && outs <= 16384)));
+  if (fixed ? tail || a.rows == 4 || K > 128 : tail && a.rows == 4) return true;
   return static_cast<int64_t>(a.rows) * K >= 1024;
 }
 

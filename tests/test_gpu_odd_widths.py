@@ -23,8 +23,9 @@ SHAPES = [(2, 9, 33), (3, 1025, 70), (5, 4098, 64), (8, 1031, 130), (13, 516, 95
 
 
 # both sides of the integer modes' choice between dot products and matrix cores, one to four rows
-FEW = [(1, 1023, 40), (1, 1025, 40), (1, 1026, 16390), (1, 2559, 40), (1, 2561, 40), (1, 4098, 16390), (1, 13900, 8200),
-       (2, 511, 70), (2, 513, 70), (2, 514, 16390), (2, 1025, 70), (3, 255, 70), (3, 257, 70), (3, 343, 70), (4, 66, 70),
+FEW = [(1, 1023, 40), (1, 1025, 40), (1, 1026, 16390), (1, 1032, 16390), (1, 2559, 40), (1, 2561, 40), (1, 2570, 16390),
+       (1, 2576, 16390), (1, 4098, 16390), (1, 13900, 8200), (2, 511, 70), (2, 512, 70), (2, 513, 70), (2, 514, 16390),
+       (2, 520, 16390), (2, 560, 70), (3, 120, 70), (3, 127, 70), (3, 136, 70), (3, 343, 70), (4, 66, 70), (4, 64, 70),
        (4, 257, 70), (3, 66, 49160)]
 
 
@@ -54,9 +55,9 @@ def test_bitlinear_odd(eng, oracle, rows, K, N, mode):  # noqa: F811
 
 
 # (rows, K, N) around the plan's limits on splitting K: 144 stages of 64 elements (K 9216, then
-# chains in steps of 16 positions) with at most 40 rows of eight 64 x 128 tiles, and 216 stages (K
-# 13824) whatever the tiles; partial tiles, tails, and the 64- and 128-row tiles split
-SPLIT = [(2, 9223, 70), (3, 9224, 70), (40, 9230, 1024), (41, 9230, 1024), (17, 9345, 1025), (40, 13831, 40),
+# chains in steps of 16 positions) with at most 40 rows of eight 64 x 128 tiles or 16 of 14, and 216
+# stages (K 13824) whatever the tiles; partial tiles, tails, and the 64- and 128-row tiles split
+SPLIT = [(2, 9223, 70), (3, 9224, 70), (40, 9230, 1024), (41, 9230, 1024), (17, 9345, 1025), (16, 9345, 1030), (16, 9345, 1800), (40, 13831, 40),
          (5, 13832, 40), (40, 14003, 333), (100, 16384, 64), (200, 13900, 700)]
 
 
