@@ -225,7 +225,7 @@ hipError_t launch_gemm_mfma(const GemmArgs& a, const ActBuf& act, hipStream_t s)
 // [nmat][rows][N] (integer modes): what the GEMM's epilogue does after its own matmul.
 hipError_t launch_acc_epilogue(const GemmArgs& a, const ActBuf& act, hipStream_t s);
 // Float mode on the fp32 matrix cores (mmf_mfma_f.hip), bit-exact with the FMA chains;
-// used when mfma_f_ok(a) and the launch has more outputs than the vector-ALU kernel takes.
+// used when mfma_f_ok(a) and the launch is past the vector-ALU kernel's line.
 bool mfma_f_ok(const GemmArgs& a);
 hipError_t launch_gemm_mfma_f(const GemmArgs& a, const ActBuf& act, hipStream_t s);
 
