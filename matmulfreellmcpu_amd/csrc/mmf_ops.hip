@@ -2256,7 +2256,8 @@ static hipError_t gemm_f_inst(const GemmArgs& a, const ActBuf& act, hipStream_t 
 // 64-16384, 16-96000 outputs per row): 8 x 2560 x 32000 {1, 1} 49.7, {2, 1} 40.5, {4, 2} 37.4; 6 x 2560 x 32000
 // {2, 2} 32.9, {4, 2} with two of eight rows idle 37.2; 3 x 2560 x 5632 x 3 {1, 1} 18.1, {2, 1} 19.0; two
 // rows a block against one, by the launch's waves at K 512 - 2000: 1536-2560 1.00x, 2560-3072 1.05x,
-// 3072-4096 1.08x; two outputs per lane and one row only for short chains (3 x 64 x 32000 {1, 1} 8.9, {1,
+// 3072-4096 1.08x (a swiglu pair, which has no {2, 1}, from 1536: 16 x 1024 x 5632 {1, 2} 13.2, {2, 2} 12.0, matrix
+// cores 13.0; 8 rows 9.8, 10.0); two outputs per lane and one row only for short chains (3 x 64 x 32000 {1, 1} 8.9, {1,
 // 2} 8.1) and rows too long for two (12 x 12000 x 5632 80 -> 77), else level.
 struct FvForm {
   int R, NO;
@@ -2270,7 +2271,9 @@ static FvForm gemm_f_form(const GemmArgs& a, const ActBuf& act) {
   for (const FvForm& f : forms) {
     const int pad = (a.rows + f.R - 1) / f.R * f.R - a.rows;
     const bool fits = f.R == 1 ? act.K < 512 || 2 * row_lds > 80 * 1024 : f.R * row_lds <= 80 * 1024;
-    if (fits && (!pair || f.NO == 2) && f.idle * pad <= a.rows && gemm_f_waves(a, f.R, f.NO) >= f.waves) return f;
+    const int64_t waves = pair && f.R == 2 ? 1536 : f.waves;
+    const int idle = pair && f.R == 2 ? 6 : f.idle;
+    if (fits && (!pair || f.NO == 2) && idle * pad <= a.rows && gemm_f_waves(a, f.R, f.NO) >= waves) return f;
   }
   return FvForm{1, pair ? 2 : 1, 0, 1};
 }
