@@ -330,6 +330,21 @@ __global__ __launch_bounds__(64 * WM * WN * KW, (mfma_min_waves<MODE, EPI, WM, W
 #pragma unroll
     for (int i = 0; i < DB; ++i) lds_dma4(brsrc, boff[i], sg * 256 * KQ, lds_addr(sb + SA + (wave * DB + i) * 256));
   };
+  // One K-group (the long-prefill tiles): this lane's operand addresses in each slot, held in
+  // registers. Left to the compiler, every stage adds them up between its barrier and its first
+  // read (3 x 2048 x 2048 of 2048 rows, FixedQ510, 53.6 us, held 53.0; K-group tiles measured 2% slower with them held).
+  constexpr int HA = KW == 1 ? D : 1;
+  uint32_t la[HA], lb[HA];
+  if constexpr (KW == 1) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      la[d] = lds_addr(ring + d * QB + wm * FM * KQ * 1024) + lane * 16;
+      lb[d] = lds_addr(ring + d * QB + SA + wn * FN * KQ * 256) + lane * 4;
+      asm volatile("" : "+v"(la[d]), "+v"(lb[d]));
+    }
+  }
+  typedef const __attribute__((address_space(3))) uint32_t lds_u32;
+  typedef const __attribute__((address_space(3))) v4i lds_v4i;
   auto stage = [&](auto sc, int st) {
     constexpr int S = decltype(sc)::value;
     // this wave's reads of the previous stage have returned and its transfers of stage st
@@ -361,15 +376,19 @@ __global__ __launch_bounds__(64 * WM * WN * KW, (mfma_min_waves<MODE, EPI, WM, W
 #pragma unroll
     for (int kh = 0; kh < KQ; ++kh)
 #pragma unroll
-      for (int bj = 0; bj < FN; ++bj)
-        bw[kh][bj] = *reinterpret_cast<const uint32_t*>(sb + SA + ((wn * FN + bj) * KQ + kh) * 256 + lane * 4);
+      for (int bj = 0; bj < FN; ++bj) {
+        if constexpr (KW == 1) bw[kh][bj] = *reinterpret_cast<lds_u32*>(lb[S] + (bj * KQ + kh) * 256);
+        else bw[kh][bj] = *reinterpret_cast<const uint32_t*>(sb + SA + ((wn * FN + bj) * KQ + kh) * 256 + lane * 4);
+      }
 #pragma unroll
     for (int kh = 0; kh < KQ; ++kh)
 #pragma unroll
       for (int pl = 0; pl < P; ++pl)
 #pragma unroll
-        for (int ai = 0; ai < FM; ++ai)
-          av[kh][pl][ai] = *reinterpret_cast<const v4i*>(sb + ((pl * FR + wm * FM + ai) * KQ + kh) * 1024 + lane * 16);
+        for (int ai = 0; ai < FM; ++ai) {
+          if constexpr (KW == 1) av[kh][pl][ai] = *reinterpret_cast<lds_v4i*>(la[S] + ((pl * FR + ai) * KQ + kh) * 1024);
+          else av[kh][pl][ai] = *reinterpret_cast<const v4i*>(sb + ((pl * FR + wm * FM + ai) * KQ + kh) * 1024 + lane * 16);
+        }
     // all LDS reads of the stage first, then the matrix-core work: each product waits only
     // for its own operands while the later reads are in flight. A group past its run (an
     // uneven split) multiplies zero weights instead of branching around the products: a
