@@ -332,7 +332,7 @@ __global__ __launch_bounds__(64 * WM * WN * KW, (mfma_min_waves<MODE, EPI, WM, W
   };
   // One K-group (the long-prefill tiles): this lane's operand addresses in each slot, held in
   // registers. Left to the compiler, every stage adds them up between its barrier and its first
-  // read (3 x 2048 x 2048 of 2048 rows, FixedQ510, 53.6 us, held 53.0; K-group tiles measured 2% slower with them held).
+  // read (3 x 2048 x 2048 of 2048 rows, FixedQ510, 53.6 us, held 52.7; K-group tiles measured 2% slower with them held).
   constexpr int HA = KW == 1 ? D : 1;
   uint32_t la[HA], lb[HA];
   if constexpr (KW == 1) {
